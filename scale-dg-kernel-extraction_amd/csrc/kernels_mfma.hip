@@ -10,7 +10,8 @@
 // Lift faces form one GEMM over the block's "pencils" r (node lines along d):
 //   out_d(r, c) = sum_l E_d F_d(r, l) D(c, l)
 //               + l-(c) flux(face d-, r) + l+(c) flux(face d+, r)
-// i.e. A_d = [E_d F_d | flux_d- | flux_d+ | 0]  (pencils x KPAD),
+// i.e. A_d = [E_d F_d | flux_d- | flux_d+ | 0]  (pencils x KPAD, the zeros
+//            supplied by the operand read),
 //      B   = [D^T ; l- ; l+ ; 0]               (KPAD x NQ), the same for
 // every direction and element.  The reference's face-node order (Fmask,
 // mod_mesh.f90:278-324) is the pencil order of the face's normal direction,
@@ -24,7 +25,9 @@
 //      registers (coalesced along (i,j));
 //   2. FP64 upwind fluxes and FP64 volume fluxes E_d q u_d, each rounded once
 //      to the operand precision, are written into augmented A arrays in LDS,
-//      one pencil per row of KPAD values;
+//      one pencil per row of an odd number of values (bank conflicts were 64%
+//      of the LDS cycles of the p = 7 mixed and p = 15 FP64 kernels, 79% at
+//      p = 18, with rows of KPAD values);
 //   3. MFMA over 16-pencil tiles; K is permuted so that lane (col, kq) keeps
 //      rows l = kq*KSTEPS + ks of B in registers and reads A at fixed offsets
 //      from its own base; the result overwrites the tile's rows in place;
@@ -105,16 +108,36 @@ struct MP {
   static constexpr int KAUG = NQ + 2;
   static constexpr int KSTEPS = (KAUG + 3) / 4;
   static constexpr int KPAD = 4 * KSTEPS;
-  static constexpr int AREA = ROWS * KPAD;                  // operands per direction
   static constexpr int NAREA = SEQ ? 1 : 3;
-  static constexpr size_t A_BYTES = (size_t)NAREA * AREA * sizeof(typename P::op_t);
+  // Operands per row of A in LDS: KAUG rounded up to odd, so that the lanes
+  // that write and read A at a stride of one row (the y and z pencils, the
+  // flux columns, the 16 rows of an MFMA operand read) spread over the banks.
+  // The K padding is not stored: the operand read puts zeros there.  KAUG
+  // itself for FP32 at p = 7, 15, where a stride of 2 (mod 8) lets the operand
+  // reads (K ranges of 3 and 5) fall into other banks too (a count of bank
+  // cycles per workgroup gives 384 and 2624 against 444 and 3056; 560 and 3776
+  // with rows of KPAD), and where the odd stride would not fit in a CU's LDS
+  // (FP64 p = 17).
+  static constexpr size_t area_bytes(int stride) {
+    return ((size_t)NAREA * ROWS * stride + 4) * sizeof(typename P::op_t);  // + read overrun
+  }
+  static constexpr bool EVEN_STRIDE = sizeof(typename P::op_t) == 4 && NQ % 8 == 0;
+  static constexpr int STRIDE =
+      !EVEN_STRIDE && area_bytes(KAUG | 1) <= 160 * 1024 ? (KAUG | 1) : KAUG;
+  static constexpr int AREA = ROWS * STRIDE;                // operands per direction
+  static constexpr size_t A_BYTES = (area_bytes(STRIDE) + 7) / 8 * 8;
   // One-wavefront all-at-once shapes first pass the q, u, v columns through
   // LDS, where each lane picks up its own x/y face traces (same area as A,
   // used before it); the others load those traces from global memory (the
   // exchange would cost them registers and a wave per SIMD)
   static constexpr bool XCH = !SEQ && WAVES == 1;
+  // k-slabs of the exchange buffers: a slab apart by one (q, u) or eight (v)
+  // more than the lanes, so the reads of different k fall into other banks
+  static constexpr int XLS = LANES + 1, XLV = LANES + 8;
   static constexpr size_t XCH_BYTES =
-      XCH ? (size_t)LANES * NQ * (sizeof(double) + 2 * sizeof(typename P::vel_t)) : 0;
+      XCH ? (size_t)NQ * (XLS * (sizeof(double) + sizeof(typename P::vel_t)) +
+                          XLV * sizeof(typename P::vel_t))
+          : 0;
   // Multi-wavefront all-at-once shapes up to p = 9: the face lanes put the
   // x/y face traces into a buffer after the A area, and the x/y fluxes are
   // formed after the barrier that already precedes the GEMMs (one barrier
@@ -181,16 +204,21 @@ constexpr int kind_of(int c) {
   return -1;
 }
 
-// One 16-pencil tile: A rows from `tile`, B (NT column tiles) in registers;
-// all A values are read before any result overwrites the tile's first NQ
-// columns.
-template <class P, int KSTEPS, int KPAD, int NQ, int NT>
+// One 16-pencil tile: A rows (STRIDE operands apart) from `tile`, B (NT column
+// tiles) in registers; all A values are read before any result overwrites the
+// tile's first NQ columns.  `left` = KAUG - kq * KSTEPS: operands of this
+// lane's K range from there on are padding, read as whatever follows the row
+// and replaced by zero.
+template <class P, int KSTEPS, int KAUG, int STRIDE, int NQ, int NT>
 __device__ __forceinline__ void mfma_tile(typename P::op_t *tile,
                                           const typename P::op_t (&bop)[NT][KSTEPS], int rd,
-                                          int wr, int col) {
+                                          int wr, int col, int left) {
   typename P::op_t a[KSTEPS];
 #pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) a[ks] = tile[rd + ks];
+  for (int ks = 0; ks < KSTEPS; ++ks) {
+    const typename P::op_t v = tile[rd + ks];
+    a[ks] = 3 * KSTEPS + ks < KAUG || ks < left ? v : (typename P::op_t)0;
+  }
   typename P::acc_t acc[NT];
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -202,7 +230,7 @@ __device__ __forceinline__ void mfma_tile(typename P::op_t *tile,
   for (int nt = 0; nt < NT; ++nt) {
     if (16 * nt + col < NQ) {
 #pragma unroll
-      for (int t4 = 0; t4 < 4; ++t4) tile[wr + 16 * nt + t4 * P::RSTRIDE_T * KPAD] = acc[nt][t4];
+      for (int t4 = 0; t4 < 4; ++t4) tile[wr + 16 * nt + t4 * P::RSTRIDE_T * STRIDE] = acc[nt][t4];
     }
   }
 }
@@ -237,7 +265,8 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
   using C = MP<P, NQ, EPB, SEQ>;
   using vel_t = typename P::vel_t;
   using op_t = typename P::op_t;
-  constexpr int NQ2 = C::NQ2, NP = C::NP, NFT = 6 * NQ2, KPAD = C::KPAD, KSTEPS = C::KSTEPS;
+  constexpr int NQ2 = C::NQ2, NP = C::NP, NFT = 6 * NQ2, KSTEPS = C::KSTEPS;
+  constexpr int KAUG = C::KAUG, STRIDE = C::STRIDE;
   constexpr int AREA = C::AREA;
   extern __shared__ double smem_mp[];
   op_t *const As = (op_t *)smem_mp;
@@ -335,14 +364,14 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
     // gathers of one cache line per two lanes on the x faces).
     if constexpr (C::XCH) {
       double *xq = (double *)smem_mp;
-      vel_t *xu = (vel_t *)(xq + C::LANES * NQ), *xv = xu + C::LANES * NQ;
+      vel_t *xu = (vel_t *)(xq + C::XLS * NQ), *xv = xu + C::XLS * NQ;
       if (active) {
 #pragma unroll
         for (int k = 0; k < NQ; ++k) {
-          xq[tid * NQ + k] = qc[k];
+          xq[k * C::XLS + tid] = qc[k];
           if constexpr (!CVEL) {
-            xu[tid * NQ + k] = uc[k];
-            xv[tid * NQ + k] = vc[k];
+            xu[k * C::XLS + tid] = uc[k];
+            xv[k * C::XLV + tid] = vc[k];
           }
         }
       }
@@ -351,8 +380,10 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
         const int src[4] = {R + i, R + (NQ - 1) + i * NQ, R + i + (NQ - 1) * NQ, R + i * NQ};
 #pragma unroll
         for (int f = 0; f < 4; ++f) {
-          qM[f] = xq[src[f] * NQ + j];
-          vM[f] = CVEL ? cv[kFaceAxis[f]] : (kFaceAxis[f] == 0 ? xu : xv)[src[f] * NQ + j];
+          qM[f] = xq[j * C::XLS + src[f]];
+          vM[f] = CVEL                  ? cv[kFaceAxis[f]]
+                  : kFaceAxis[f] == 0 ? xu[j * C::XLS + src[f]]
+                                      : xv[j * C::XLV + src[f]];
         }
       }
       __syncthreads();  // the A operands below reuse the area
@@ -435,13 +466,14 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
                       : l == NQ + 1 ? ell_[NQ + c] : (op_t)0;
       }
     }
-    const int rd = col * KPAD + kq * KSTEPS;        // A read offset of this lane in a tile
-    const int wr = P::RSTRIDE_Q * kq * KPAD + col;  // result offset of value 0
+    const int rd = col * STRIDE + kq * KSTEPS;        // A read offset of this lane in a tile
+    const int wr = P::RSTRIDE_Q * kq * STRIDE + col;  // result offset of value 0
+    const int left = KAUG - kq * KSTEPS;              // stored operands of the lane's K range
     // Node (i,j,k) sits in the x pencil (j,k) at position i, in the y pencil
     // (i,k) at position j and in the z pencil (i,j) at position k; face node
     // (i,j) of the faces normal to d is pencil ij of direction d.
-    const int pos_off[3] = {(R + j) * KPAD + i, (R + i) * KPAD + j, (R + ij) * KPAD};
-    const int pos_step[3] = {NQ * KPAD, NQ * KPAD, 1};
+    const int pos_off[3] = {(R + j) * STRIDE + i, (R + i) * STRIDE + j, (R + ij) * STRIDE};
+    const int pos_step[3] = {NQ * STRIDE, NQ * STRIDE, 1};
     // non-temporal RK base and output where k-slabs are whole 128-byte lines;
     // cached where one instruction covers pieces of lines (p <= 6), so the L2
     // merges them (as stage_f64; mixed p = 2, 4: 6% faster per launch)
@@ -462,13 +494,11 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
             const vel_t vel = d == 0 ? uc[k] : d == 1 ? vc[k] : wc[k];
             a[k * pos_step[d]] = (op_t)(Ed * (qc[k] * (double)vel));
           }
-          op_t *r = As + d * AREA + (R + ij) * KPAD;
+          op_t *r = As + d * AREA + (R + ij) * STRIDE;
           if (!C::XD || d == 2) {
             r[NQ] = fl[face_m[d]];
             r[NQ + 1] = fl[face_p[d]];
           }
-#pragma unroll
-          for (int l = NQ + 2; l < KPAD; ++l) r[l] = (op_t)0;
         }
       }
       // RK base column, in flight during the GEMMs (the RK base and the output
@@ -490,7 +520,7 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
           }
 #pragma unroll
           for (int d = 0; d < 2; ++d) {
-            op_t *r = As + d * AREA + (R + ij) * KPAD;
+            op_t *r = As + d * AREA + (R + ij) * STRIDE;
             r[NQ] = fl[face_m[d]];
             r[NQ + 1] = fl[face_p[d]];
           }
@@ -506,7 +536,8 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
         const int job = wave + jj * C::WAVES;
         if (job >= C::JOBS) break;  // wave-uniform
         const int d = job / C::MTILES, t = job - d * C::MTILES;
-        mfma_tile<P, KSTEPS, KPAD, NQ, NT>(As + d * AREA + t * 16 * KPAD, bop, rd, wr, col);
+        mfma_tile<P, KSTEPS, KAUG, STRIDE, NQ, NT>(As + d * AREA + t * 16 * STRIDE, bop, rd, wr,
+                                                   col, left);
       }
       __syncthreads();
 
@@ -530,18 +561,16 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
           for (int k = 0; k < NQ; ++k)
             a[k * pos_step[d]] =
                 (op_t)(Ed * (qc[k] * (double)(CVEL ? cv[d] : vel[base + k * NQ2])));
-          op_t *r = As + (R + ij) * KPAD;
+          op_t *r = As + (R + ij) * STRIDE;
           r[NQ] = fl[face_m[d]];
           r[NQ + 1] = fl[face_p[d]];
-#pragma unroll
-          for (int l = NQ + 2; l < KPAD; ++l) r[l] = (op_t)0;
         }
         __syncthreads();
 #pragma unroll
         for (int jj = 0; jj < C::JPW; ++jj) {
           const int t = wave + jj * C::WAVES;
           if (t >= C::MTILES) break;  // wave-uniform
-          mfma_tile<P, KSTEPS, KPAD, NQ, NT>(As + t * 16 * KPAD, bop, rd, wr, col);
+          mfma_tile<P, KSTEPS, KAUG, STRIDE, NQ, NT>(As + t * 16 * STRIDE, bop, rd, wr, col, left);
         }
         __syncthreads();
         if (active) {
@@ -831,7 +860,7 @@ stage_run_mp(const double *__restrict__ q_, const double *q0_, const float *__re
     const int job = wave + jj * C::WAVES;
     if (job >= C::JOBS) break;  // wave-uniform
     const int d = job / C::MTILES, t = job - d * C::MTILES;
-    mfma_tile<P, KSTEPS, KPAD, NQ, 1>(As + d * AREA + t * 16 * KPAD, bop, rd, wr, col);
+    mfma_tile<P, KSTEPS, KPAD, KPAD, NQ, 1>(As + d * AREA + t * 16 * KPAD, bop, rd, wr, col, KPAD);
   }
   __syncthreads();
 
@@ -1006,13 +1035,16 @@ std::atomic<int> g_mp_shape[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
 // same timings with the velocity read from the geometry record, among the
 // shapes that give the bits of the default above (the MFMA shapes and the
 // run kernel), so a served request equals its solve on a plain solver: two
-// wavefronts at p = 3 (161 -> 152 us), one wavefront at p = 5 (119 -> 105 us),
-// the direction-by-direction shape at p = 6, 9, 12 (109 -> 102, 105 -> 98,
-// 112 -> 106 us).
-constexpr int kMpDefaultCvel[kMaxNq + 1] = {0, 0, 5, 0, 1, 1, 0, 3, 0, 0, 2,
-                                            0, 0, 2, 0, 2, 0, 1, 1, 0, 0};
-std::atomic<int> g_mp_shape_cvel[kMaxNq + 1] = {0, 0, 5, 0, 1, 1, 0, 3, 0, 0, 2,
-                                                0, 0, 2, 0, 2, 0, 1, 1, 0, 0};
+// wavefronts at p = 2, 3 (183 -> 161 and 150 -> 148 us per launch against
+// one), one wavefront at p = 5 (129 -> 108 us against two), and direction by
+// direction at p = 6, 8, 9, 11..19 where it needs a third of the LDS and no
+// velocity load sits between its directions (p = 8 105 -> 98, p = 12 101 ->
+// 99, p = 13 94 -> 89, p = 15 97 -> 90, p = 18 131 -> 110, p = 19 137 ->
+// 119 us).
+constexpr int kMpDefaultCvel[kMaxNq + 1] = {0, 0, 5, 1, 1, 1, 0, 3, 0, 2, 2,
+                                            0, 2, 2, 2, 2, 2, 1, 1, 1, 1};
+std::atomic<int> g_mp_shape_cvel[kMaxNq + 1] = {0, 0, 5, 1, 1, 1, 0, 3, 0, 2, 2,
+                                                0, 2, 2, 2, 2, 2, 1, 1, 1, 1};
 
 template <class P, int NQ>
 int prepare_nq_all() {
