@@ -9,7 +9,8 @@ region.  Metric: DOF-updates/s = Ne*Np*K / t for K timed steps.
 
 The JSON line also carries
   roofline      the FP64 stage kernel: algorithmic HBM bytes per launch
-                (136/3 B per DOF) over its average launch time, from HIP events
+                (64/3 B per DOF, the wind being constant; 136/3 B with
+                DGK_CVEL=0) over its average launch time, from HIP events
                 recorded on the solver's stream around every launch; traffic
                 from the rocprofv3 FETCH_SIZE/WRITE_SIZE summary in profiles/;
   cpu_baseline  the reference Fortran GENERAL path (oracle/_ref, OpenMP on the
@@ -32,6 +33,7 @@ The JSON line also carries
 from __future__ import annotations
 
 import argparse
+import contextlib
 import csv
 import json
 import os
@@ -45,7 +47,12 @@ ROOT = Path(__file__).resolve().parent
 sys.path.insert(0, str(ROOT / "scale-dg-kernel-extraction_amd"))
 
 HBM_PEAK_GBS = 8000.0
-BYTES_PER_DOF_UPDATE = {"HIP": 136.0, "HIP_MP": 100.0}
+# The workloads' winds are constant, and the stage kernels read a constant wind
+# from the geometry record: q read and written each stage and q0 read on two.
+# DGK_CVEL=0 keeps the velocity fields' reads.
+CONSTANT_WIND = os.environ.get("DGK_CVEL", "1")[:1] != "0"
+BYTES_PER_DOF_UPDATE = ({"HIP": 64.0, "HIP_MP": 64.0} if CONSTANT_WIND
+                        else {"HIP": 136.0, "HIP_MP": 100.0})
 METRIC = "DOF-updates/s plain FP64 vs batched mixed-prec; p50/p99 solve latency"
 
 
@@ -182,7 +189,8 @@ def time_solver(dgk, inputs, form, steps, warmup, autotune=True):
     s = dgk.Solver.structured(form, wl.NeX, wl.NeY, wl.NeZ, wl.p)
     s.set_fields(wl.q, wl.u, wl.v, wl.w)
     tune = s.autotune(reps=10) if autotune else {"best": s.tile(), "us_per_launch": None}
-    tune["kernel"] = dgk.kernel_name(form, wl.p, tune["best"])
+    tune["kernel"] = dgk.kernel_name(form, wl.p, tune["best"],
+                                     constant_velocity=CONSTANT_WIND)
     s.step(wl.dt, warmup)
     s.synchronize()
     s.timer_reset()
@@ -224,6 +232,20 @@ def pcie_leg(dgk, inputs, form, steps):
     return {"form": form, "steps": steps, "DOF-updates/s": dof * steps / (t3 - t0),
             "upload_s": t1 - t0, "steps_s": t2 - t1, "download_s": t3 - t2,
             "host_bytes": 5 * dof * 8}
+
+
+@contextlib.contextmanager
+def cvel_env(value):
+    """DGK_CVEL=value while velocities are set ("0": launches read the fields)."""
+    before = os.environ.get("DGK_CVEL")
+    os.environ["DGK_CVEL"] = value
+    try:
+        yield
+    finally:
+        if before is None:
+            del os.environ["DGK_CVEL"]
+        else:
+            os.environ["DGK_CVEL"] = before
 
 
 def batch_leg(dgk, inputs):
@@ -279,7 +301,8 @@ def batch_leg(dgk, inputs):
     for k in p7:
         it = ens[k]
         s = dgk.Solver.structured("HIP", *it["ne"], it["p"])
-        s.init_gaussian(it["centre"], it["sigma"], it["vel"])
+        with cvel_env("0"):  # velocity fields, as the decomposition below counts them
+            s.init_gaussian(it["centre"], it["sigma"], it["vel"])
         s.step(it["dt"], 1)
         s.synchronize()
         t0 = time.perf_counter()
@@ -294,11 +317,8 @@ def batch_leg(dgk, inputs):
     sub = [ens[k] for k in p7]
     rates = {}
     for form, cvel in (("HIP", "0"), ("HIP", "1"), ("HIP_MP", "0"), ("HIP_MP", "1")):
-        os.environ["DGK_CVEL"] = cvel
-        try:
+        with cvel_env(cvel):
             rec, _ = run_batch(form, sub)
-        finally:
-            os.environ.pop("DGK_CVEL", None)
         key = f"batched_{form}_p7" + ("" if cvel == "1" else "_velocity_fields")
         rec["bytes_per_dof_update"] = 64 if cvel == "1" else (136 if form == "HIP" else 100)
         rec.pop("tile_shapes", None)
@@ -363,8 +383,10 @@ def per_order_only(dgk, form, p, steps):
         s.init_gaussian((0.3, 0.6, 0.2), 0.1, (0.9, -0.4, 0.3))
         s.step(0.05 * (2.0 / ne) / (p + 1), steps)
         s.synchronize()
+        tile = s.tile()
     print(json.dumps({"per_order_only": p, "form": form, "ne": ne, "dof": dof, "steps": steps,
-                      "kernel": dgk.kernel_name(form, p, dgk.tile_selected(form, p))}), flush=True)
+                      "kernel": dgk.kernel_name(form, p, tile,
+                                                constant_velocity=CONSTANT_WIND)}), flush=True)
 
 
 PER_ORDER_ORDERS = tuple(range(1, 20))
@@ -393,13 +415,14 @@ def per_order_leg(dgk, orders=PER_ORDER_ORDERS, steps=30, warmup=30):
                 s.step(dt, steps)
                 s.synchronize()
                 sec, n = s.timers()["Stage (fused)"]
+                tile = s.tile()
             launch = sec / n
             gbs = BYTES_PER_DOF_UPDATE[form] / 3.0 * dof / launch / 1e9
             tfs = flops_per_dof_update(p) / 3.0 * dof / launch / 1e12
             peak = 78.6 if form == "HIP" else 157.3
-            shape = dgk.tile_shapes(form, p)[dgk.tile_selected(form, p)]
+            shape = dgk.tile_shapes(form, p)[tile]
             out.append({"p": p, "form": form, "ne": ne, "dof": dof, "avg_launch_us": 1e6 * launch,
-                        "tile_candidate": dgk.tile_selected(form, p), "elements_per_workgroup": shape,
+                        "tile_candidate": tile, "elements_per_workgroup": shape,
                         "DOF-updates/s": dof / (3.0 * launch), "alg_GBs": gbs,
                         "frac_hbm": gbs / HBM_PEAK_GBS, "useful_TFLOPs": tfs,
                         "frac_mfma_peak": tfs / peak})
@@ -552,8 +575,9 @@ def main():
             "ratio_vs_" + args.form: r2["value"] / r["value"]}
         line["extra"]["pcie_inclusive"] = pcie_leg(dgk, inputs, args.form, args.steps)
         be = batch_leg(dgk, inputs)
+        wind = "constant velocity" if CONSTANT_WIND else "velocity fields"
         be["decomposition_p7"]["batched mixed (constant velocity) / plain FP64 headline "
-                               "(one 32^3 p=7 mesh, velocity fields)"] = (
+                               f"(one 32^3 p=7 mesh, {wind})"] = (
             be["batched_HIP_MP_p7"]["DOF-updates/s"] / line["value"])
         line["extra"]["batched_ensemble"] = be
         line["extra"]["c3_p15"] = c3_leg(dgk, inputs)

@@ -153,7 +153,13 @@ int dgk_init_gaussian(dgk_solver *s, double cx, double cy, double cz, double sig
 
 /* Upload a field, n = Np*Ne (owned part) or Np*NeA (the halo tail is
  * ignored: it is derived from the owned part).  Setting U, V or W refreshes
- * their halos once, as main.f90:160-162 does. */
+ * their halos once, as main.f90:160-162 does.  While U, V and W each
+ * hold one value over the whole mesh (bit for bit; also after
+ * dgk_init_gaussian) and the face normals lie along the axes, the stage
+ * kernels read the wind from the geometry records instead of the fields: the
+ * same bits, 64 bytes per DOF-update instead of 136 (HIP) or 100 (HIP_MP).
+ * DGK_CVEL=0 in the environment when a velocity is set keeps the field
+ * reads. */
 int dgk_set_field(dgk_solver *s, int which, const double *f, int64_t n);
 /* Download a field, n = Np*Ne or Np*NeA.  With n = Np*NeA the halo tail holds
  * what the last dgk_update_halo wrote (zeros before any). */
@@ -278,10 +284,11 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  *           direction-by-direction MFMA shape (the last candidate) at
  *           p = 14..19, the staged VALU kernel otherwise.
  * Constant-velocity launches (batch groups of constant-velocity instances,
- * served requests) start from defaults of their own, taken only among shapes
- * that give the bits of the defaults above: FP64 the register VALU kernel
- * also at p = 2, 3; mixed two wavefronts at p = 3, one at p = 5, the
- * direction-by-direction shape at p = 6, 9, 12.
+ * served requests, solvers whose velocity fields are constant) start from
+ * defaults of their own, taken only among shapes that give the bits of the
+ * defaults above: FP64 the register VALU kernel also at p = 2, 3; mixed two
+ * wavefronts at p = 2, 3, one at p = 5, the direction-by-direction shape at
+ * p = 6, 8, 9, 11..19.
  * dgk_tile_select sets the process-wide choice for that form and order, for
  * both kinds of launch (-1 restores the defaults); it holds for every solver
  * that has not been autotuned; dgk_tile_selected reports the choice for
@@ -294,8 +301,8 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * faster);
  * us_per_launch[c] receives candidate c's time (0 for a candidate that would
  * launch another shape on this solver: the kernel over runs of elements, on
- * launches it cannot take -- constant velocities, a resolved face-node table,
- * an explicit order).  dgk_batch_autotune does this
+ * launches it cannot take -- batches' constant velocities, a resolved face-node
+ * table, an explicit order).  dgk_batch_autotune does this
  * for every order group of a batch and reports per group: the order, the
  * chosen candidate, its time and the default's time (the batch's captured
  * step is re-captured at the next dgk_batch_step).  No counterpart

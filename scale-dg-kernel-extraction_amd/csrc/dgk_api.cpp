@@ -147,6 +147,27 @@ int refresh_f32(dgk_solver *s, int which) {
   return launch_to_f32(field_ptr(s, which), dst, (int64_t)s->Np * s->Ne, s->stream);
 }
 
+static int geo_velocity_from_field(dgk_solver *s, int d) {
+  // the mixed form's fields are FP32 copies: the record holds the same value
+  return launch_geo_velocity(s->geo, s->ngeo, d, field_ptr(s, DGK_FIELD_U + d),
+                             s->evaltype == DGK_EVAL_HIP_MP, s->stream);
+}
+
+// The kind of the solver's stage launches after a change of its velocity
+// fields: constant components on axis-aligned faces are read from the
+// geometry records, 64 bytes per DOF-update instead of 136 (FP64) or 100
+// (mixed), with the same bits (at 32^3, p = 7: 139 -> 101 us per launch FP64,
+// 102 -> 94 us mixed).  Node connectivity has no such form.  DGK_CVEL=0 keeps
+// the per-node reads (for A/B timings).  A tile shape autotuned for one kind
+// is kept for it.
+static void choose_velocity_form(dgk_solver *s) {
+  const char *env = std::getenv("DGK_CVEL");
+  const bool all = s->vel_constant[0] && s->vel_constant[1] && s->vel_constant[2];
+  const int cvel = all && s->axis_aligned && !s->vmapP && !(env && env[0] == '0') ? 2 : 0;
+  if (cvel != s->cvel) std::swap(s->tile, s->tile_other);
+  s->cvel = cvel;
+}
+
 // Backwards launches walk each XCD's own slot range backwards where the
 // order is XCD-interleaved: an XCD then starts a launch on the elements it
 // ended the previous one with (per launch at about 1.7e7 DOF, against
@@ -278,6 +299,7 @@ int create_from_tables(int evaltype, MeshTables &t, dgk_solver **out) {
   s->Ne = t.Ne; s->NeA = t.NeA; s->NhaloNode = t.NhaloNode;
   s->nfield = (int64_t)t.Np * t.Ne + t.NhaloNode;
   s->axis_aligned = t.axis_aligned ? 1 : 0;
+  s->ngeo = (int64_t)(t.geo.size() / kGeoStride);
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess)
     return fail(set_error(DGK_ERR_DEVICE, "hipStreamCreate failed"));
   for (int b = 0; b < 3; ++b)
@@ -429,6 +451,11 @@ int dgk_init_gaussian(dgk_solver *s, double cx, double cy, double cz, double sig
     DGK_TRY(refresh_f32(s, which));
   }
   for (int f = 0; f < 4; ++f) s->set[f] = true;
+  for (int d = 0; d < 3; ++d) {
+    DGK_TRY(geo_velocity_from_field(s, d));
+    s->vel_constant[d] = true;
+  }
+  choose_velocity_form(s);
   s->q0_valid = s->flux_valid = s->dqdt_valid = false;
   DGK_HIP(hipStreamSynchronize(s->stream));
   return DGK_OK;
@@ -478,10 +505,28 @@ int dgk_set_field(dgk_solver *s, int which, const double *f, int64_t n) {
   if (n != owned && n != (int64_t)s->Np * s->NeA)
     return set_error(DGK_ERR_ARG, "field length must be Np*Ne or Np*NeA");
   double *dst = field_ptr(s, which);
+  if (which != DGK_FIELD_Q) {
+    s->vel_constant[which - DGK_FIELD_U] = false;  // until the new field has been looked at
+    choose_velocity_form(s);
+  }
   DGK_HIP(hipMemcpyAsync(dst, f, sizeof(double) * owned, hipMemcpyHostToDevice, s->stream));
   if (which != DGK_FIELD_Q) {
     DGK_TRY(launch_halo_gather(dst, s->halo, owned, s->NhaloNode, s->stream));
     DGK_TRY(refresh_f32(s, which));
+    // one value everywhere?  The device looks only if a few values agree.
+    const int d = which - DGK_FIELD_U;
+    int32_t varies = 0;
+    for (int64_t k : {owned / 3, owned / 2, owned - 1})
+      varies |= std::memcmp(f + k, f, sizeof(double)) != 0;
+    if (!varies) {
+      int32_t *flag = (int32_t *)s->mm;
+      DGK_TRY(launch_varies(dst, owned, flag, s->stream));
+      DGK_HIP(hipMemcpyAsync(&varies, flag, sizeof(varies), hipMemcpyDeviceToHost, s->stream));
+      DGK_TRY(geo_velocity_from_field(s, d));
+    }
+    DGK_HIP(hipStreamSynchronize(s->stream));
+    s->vel_constant[d] = !varies;
+    choose_velocity_form(s);
   } else {
     s->q0_valid = false;
   }

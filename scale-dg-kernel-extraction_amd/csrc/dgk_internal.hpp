@@ -247,7 +247,8 @@ struct StageArgs {
   int tile;               // tile-shape candidate, -1: the process-wide selection
   int geo_per_run = 0;    // with geoid: every run of run_elements(Nq) elements from a
                           // multiple of it shares one geometry record
-  int cvel = 0;           // velocity constant per element, from its geometry record
+  int cvel = 0;           // velocity constant per element, from its geometry record; 2: the
+                          // fields hold it too, for kernels that read fields only
 };
 
 // Mixed-precision operands (FP32 copies of the constant inputs).
@@ -327,6 +328,11 @@ int launch_rk_update(double *q, const double *q0, const double *dqdt,
 int launch_minmax(const double *q, int64_t n, double *partial, int nblk,
                   double *result, hipStream_t s);
 int launch_to_f32(const double *src, float *dst, int64_t n, hipStream_t s);
+// *flag = 1 if some f[t] differs (bit for bit) from f[0], else 0.
+int launch_varies(const double *f, int64_t n, int32_t *flag, hipStream_t s);
+// Word kGeoVel + d of ngeo geometry records = f[0], rounded to FP32 with f32.
+int launch_geo_velocity(double *geo, int64_t ngeo, int d, const double *f, bool f32,
+                        hipStream_t s);
 int launch_init_gaussian(double *q, double *u, double *v, double *w, const double *x1D,
                          int Nq, int NeX, int NeY, int NeZ, const double h[3],
                          const double c[3], double sigma, const double vel[3],

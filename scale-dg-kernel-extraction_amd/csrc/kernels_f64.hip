@@ -839,6 +839,23 @@ __global__ void to_f32(const double *__restrict__ src, float *__restrict__ dst,
   if (t < n) dst[t] = (float)src[t];
 }
 
+// One pass over a field that may be constant; bound by the read (134 MB of a
+// 32^3 mesh at p = 7 in about 30 us, against 6 ms for its upload).
+__global__ void varies(const uint64_t *__restrict__ f, int64_t n, int32_t *flag) {
+  const uint64_t f0 = f[0];
+  bool d = false;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n;
+       t += (int64_t)gridDim.x * blockDim.x)
+    d |= f[t] != f0;
+  if (d) *flag = 1;
+}
+
+__global__ void geo_velocity(double *geo, int64_t ngeo, int d, const double *__restrict__ f,
+                             int f32) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < ngeo) geo[r * kGeoStride + kGeoVel + d] = f32 ? (double)(float)f[0] : f[0];
+}
+
 unsigned grid1d(int64_t n, int threads) {
   return (unsigned)((n + threads - 1) / threads);
 }
@@ -1107,6 +1124,24 @@ int launch_init_gaussian(double *q, double *u, double *v, double *w, const doubl
 int launch_to_f32(const double *src, float *dst, int64_t n, hipStream_t s) {
   if (n == 0) return DGK_OK;
   hipLaunchKernelGGL(to_f32, dim3(grid1d(n, 256)), dim3(256), 0, s, src, dst, n);
+  DGK_HIP(hipGetLastError());
+  return DGK_OK;
+}
+
+int launch_varies(const double *f, int64_t n, int32_t *flag, hipStream_t s) {
+  DGK_HIP(hipMemsetAsync(flag, 0, sizeof(int32_t), s));
+  if (n == 0) return DGK_OK;
+  hipLaunchKernelGGL(varies, dim3(std::min(grid1d(n, 256), 4096u)), dim3(256), 0, s,
+                     (const uint64_t *)f, n, flag);
+  DGK_HIP(hipGetLastError());
+  return DGK_OK;
+}
+
+int launch_geo_velocity(double *geo, int64_t ngeo, int d, const double *f, bool f32,
+                        hipStream_t s) {
+  if (ngeo == 0) return DGK_OK;
+  hipLaunchKernelGGL(geo_velocity, dim3(grid1d(ngeo, 256)), dim3(256), 0, s, geo, ngeo, d, f,
+                     f32 ? 1 : 0);
   DGK_HIP(hipGetLastError());
   return DGK_OK;
 }

@@ -923,7 +923,7 @@ bool aligned16_mp(const void *p) { return ((uintptr_t)p & 15) == 0; }
 // within a tile, unaligned fields, or constant velocities (no fields).
 bool run_mp_applicable(int Nq, const StageArgsMP &a) {
   const int T = run_mp_elements(Nq);
-  if (T < 1 || !a.nbr || a.vmapP || a.order || a.cvel) return false;
+  if (T < 1 || !a.nbr || a.vmapP || a.order || a.cvel == 1) return false;
   if (a.geoid && !a.geo_per_run) return false;
   const bool q0_ok = a.mode != 1 || a.ca == 0.0 || aligned16_mp(a.q0);
   return aligned16_mp(a.q) && aligned16_mp(a.u) && aligned16_mp(a.v) && aligned16_mp(a.w) &&

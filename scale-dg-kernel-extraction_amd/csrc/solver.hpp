@@ -43,7 +43,11 @@ struct dgk_solver {
   int tile = -1;             // tile-shape candidate chosen for this mesh (-1: process default)
   int geo_per_run = 1;       // every run of run_elements(Nq) elements shares a geometry record
   int cvel = 0;              // stage launches read each element's constant velocity from its
-                             // geometry record (batch groups whose boxes all have one)
+                             // geometry record (1: batch groups whose boxes all have one, served
+                             // requests; 2: a solver whose velocity fields are constant)
+  bool vel_constant[3] = {false, false, false};  // u, v, w hold one value each
+  int tile_other = -1;       // `tile` of the other kind of launch (fields / constant velocity)
+  int64_t ngeo = 0;          // geometry records
   double *x1D = nullptr;     // LGL nodes (device), for device-side initial conditions
   BoxShape box;              // structured box (NeX == 0 when built from arrays)
   int32_t *nbr = nullptr, *vmapP = nullptr, *halo = nullptr;
