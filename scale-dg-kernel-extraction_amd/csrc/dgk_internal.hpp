@@ -124,6 +124,11 @@ __device__ __forceinline__ int64_t slot_element(int64_t slot, int64_t Ne,
   }
   return slot;
 }
+// Ex dx + Ey dy, with the fused product fixed: the FP64 VALU kernels and the
+// run kernel give the same bits whatever the code around it.
+__device__ __forceinline__ double combine_xy(double Ex, double dx, double Ey, double dy) {
+  return __builtin_fma(Ex, dx, Ey * dy);
+}
 template <int NQ>
 __device__ __forceinline__ int64_t nbr_node(bool resolved, int32_t t, int f, int i, int j) {
   return resolved ? (int64_t)t : (int64_t)t * (NQ * NQ * NQ) + nbr_face_node(f, i, j, NQ);

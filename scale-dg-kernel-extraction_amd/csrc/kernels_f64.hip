@@ -28,6 +28,9 @@
 //      from the stored Lift_mat (checked separable at solver creation) -- and
 //      dqdt = -(((Ex Dx + Ey Dy) + Ez Dz) + Lift), stored or RK-combined.
 //
+// With axis-aligned faces and no given flux the register form (VREG) runs
+// stage_pencil instead: the same arithmetic, a pencil per lane and direction.
+//
 // stage_f64_lift<NQ> (stored Lift): the same arithmetic with Lift_mat read as
 // stored; used when Lift_mat is not of tensor-product form.
 #include <algorithm>
@@ -91,12 +94,6 @@ struct Staged {
   // register form at p = 11, which otherwise lands one VGPR above the
   // 168 that 3 waves allow (and drops to 2).
   static constexpr int MIN_WAVES_EU = (VREG && NQ == 12) ? 3 : 1;
-  // The axis-aligned register form also at p = 3, 4 (5 waves: 100 and 118
-  // VGPRs -> 83-92, no spills; launches 6% faster) and p = 13 (3 waves: 183
-  // VGPRs -> 168 with 28 bytes per lane spilled; 4% faster).  The staged
-  // form ran slower held the same way.
-  static constexpr int MIN_WAVES_EU_AX = !VREG ? 1 : NQ == 12 ? 3 : (NQ == 4 || NQ == 5) ? 5
-                                         : NQ == 14 ? 3 : 1;
 };
 
 // AXAL: every face normal lies along its face's axis (checked on the host), so
@@ -104,8 +101,7 @@ struct Staged {
 // other components enter the normal velocity as exact zeros).  The general
 // form holds three more traces per face in registers; a compile-time choice
 // lets the axis-aligned kernel drop them (p = 1: 85 -> 62 VGPRs, 5 -> 8 waves
-// per SIMD).  The register form at p = 11 keeps the test at run time: with
-// it decided at compile time the allocation lands at 168 VGPRs with 2 spilled.
+// per SIMD).  The axis-aligned register forms run stage_pencil instead.
 // CVEL: every element's velocity is constant, (u, v, w) = words kGeoVel..+2
 // of its geometry record (batched and served boxes); no velocity field is
 // read.  The constants enter the same expressions as the per-node values
@@ -127,7 +123,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
            const double *__restrict__ ell_, const double *__restrict__ geo_,
            const uint32_t *__restrict__ geoid_, const int32_t *__restrict__ order_,
            const int64_t Ne_, const double ca_, const double cb_, const double dt_,
-           const int mode_, const int axis_aligned_, const int dt_geo_, const int rev_,
+           const int mode_, const int dt_geo_, const int rev_,
            const int64_t zp_) {
   // Read-only operands are __restrict__ kernel parameters, so wave-uniform
   // reads of them (operators, geometry, neighbour table) are scalar loads.
@@ -245,8 +241,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
     // neighbour traces of face node (i,j) on all six faces, and the RK base
     // column, in flight together with the async copy (axis-aligned: q and the
     // normal velocity component, fixed per face at compile time)
-    constexpr bool AX_RUNTIME = VREG && NQ == 12;
-    const bool axal = AX_RUNTIME ? axis_aligned_ != 0 : AXAL;
+    constexpr bool axal = AXAL;
     double qP[6], uP[6], vP[6], wP[6], q0v[NQ];
     if (active && !flux_in_) {
       auto nbr_at = [&](int f) -> int64_t {
@@ -391,7 +386,292 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
         const double lift = lmj * G[0 * NQ2 + i + k * NQ] + lpi * G[1 * NQ2 + j + k * NQ] +
                             lpj * G[2 * NQ2 + i + k * NQ] + lmi * G[3 * NQ2 + j + k * NQ] +
                             sL[k] * gf[4] + sL[NQ + k] * gf[5];
-        const double tend = -(((Ex * dx + Ey * dy) + Ez * dz) + lift);
+        const double tend = -((combine_xy(Ex, dx, Ey, dy) + Ez * dz) + lift);
+        const int64_t idx = base + (int64_t)k * NQ2;
+        double res = tend;
+        if (rk) {
+          const double upd = cb_ * (qc[k] + (dt_geo_ ? g[kGeoDt] : dt_) * tend);
+          res = use_q0 ? ca_ * q0v[k] + upd : upd;
+        }
+        if constexpr (NT_SLAB) __builtin_nontemporal_store(res, out_ + idx);
+        else out_[idx] = res;
+      }
+    }
+  };
+  if constexpr (GU) body(geo_);
+  else body(g_lane);
+}
+
+// acc[c] = sum over l (ascending) of D(c, l) F[l], D read through the scalar
+// cache one column ahead.  The address of column l + 1 is made opaque at a
+// point that follows column l - 1's arithmetic: otherwise the compiler loads
+// all NQ columns first, and the 2 NQ^2 scalar registers spill.
+typedef const double __attribute__((address_space(4))) *uniform_ptr;
+template <int NQ>
+__device__ __forceinline__ void contract(const double *D, const double (&F)[NQ],
+                                         double (&acc)[NQ]) {
+  uniform_ptr p = (uniform_ptr)D;
+  double cur[NQ], nxt[NQ];
+#pragma unroll
+  for (int c = 0; c < NQ; ++c) {
+    acc[c] = 0.0;
+    cur[c] = p[c];
+  }
+#pragma unroll
+  for (int l = 0; l < NQ; ++l) {
+    if (l + 1 < NQ) {
+      asm volatile("" : "+s"(p));
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) asm volatile("" : "+v"(acc[c]));
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) nxt[c] = p[c + (l + 1) * NQ];
+    }
+#pragma unroll
+    for (int c = 0; c < NQ; ++c) {
+      acc[c] += cur[c] * F[l];
+      cur[c] = nxt[c];
+    }
+  }
+}
+
+// Pencil form of the stage (axis-aligned faces, flux computed here): lane (a,b)
+// of an element owns in turn the x pencil (:,a,b), the y pencil (a,:,b) and the
+// z pencil (a,b,:).
+//   1. the lane loads its z columns of q, u (, v, w, q0) and the six neighbour
+//      traces into registers and writes q and u to LDS (rows of an odd number
+//      of doubles);
+//   2. it reads the x pencils of q and u and the y pencil of q.  Face node (a,b)
+//      of the x faces is an end of the x pencil, so the upwind fluxes need no
+//      other own trace; D applies to the pencil in registers, its entries scalar
+//      operands (contract below).  Dx goes back to LDS in place of q, v in place
+//      of u;
+//   3. the same along y; Ex Dx + Ey Dy replaces Dx;
+//   4. the same along z, Lift, RK update.
+// What bounded the form it replaced (stage_valu with v, w in registers) was the
+// LDS: 284 double accesses per node column at p = 7, of which 192 fed the three
+// contractions one operand at a time (LDS busy 52% of the cycles), and the
+// scalar loads before its first field load.  This one makes 124 (108 with a
+// constant velocity, and half the LDS).  us per launch at about 1.7e7 DOF,
+// start -> now, velocity fields: p = 4 168 -> 159, p = 7 142 -> 129, p = 8
+// 163 -> 146, p = 11 159 -> 138, p = 12 187 -> 153, p = 13 181 -> 161; a
+// solver's constant velocity (it read the fields): p = 1 187 -> 102, p = 3
+// 154 -> 77, p = 7 142 -> 74 (4.8 TB/s), p = 12 187 -> 90.  What is left with
+// fields is the streaming rate (124 us for these bytes at 6.1 TB/s) at p = 7
+// and 11, with a constant velocity the workgroup's own chain of phases.
+// Capping the registers for one more wave per SIMD spills and runs up to 2x
+// slower, except with fields at p = 13 (164 -> 158 us).
+template <int NQ, bool CVEL>
+struct Pencil {
+  static constexpr int NQ2 = NQ * NQ, NP = NQ2 * NQ;
+  static constexpr int EPB = Staged<NQ, true>::EPB, THREADS = Staged<NQ, true>::THREADS;
+  // row, slab and element strides in doubles: an odd row spreads the lanes of
+  // an x pencil read (a row apart) and of a z column write over the banks
+  static constexpr int S1 = NQ | 1, S2 = NQ * S1, SE = NQ * S2;
+  static constexpr int BUF = EPB * SE;                 // doubles of one field
+  static constexpr int OFF_G = (CVEL ? 1 : 2) * BUF;   // x/y-face fluxes [EPB][4][NQ2]
+  static constexpr int OFF_L = OFF_G + EPB * 4 * NQ2;
+  static constexpr int LDS_DOUBLES = OFF_L + 2 * NQ;
+  static constexpr size_t LDS_BYTES = sizeof(double) * LDS_DOUBLES;
+  // above p = 7 the v, w and q0 columns are loaded a phase before their use:
+  // held from the start they cost a wave per SIMD (p = 11 fields 141 -> 170 us)
+  static constexpr bool LATE = NQ > 8;
+  static constexpr int MIN_WAVES_EU = !CVEL && NQ == 14 ? 3 : 1;
+  // Non-temporal RK base and output: with velocity fields where a k-slab is
+  // whole 128-byte lines and above p = 8 (p = 7 135 -> 129 us, p = 15 172 ->
+  // 160); cached elsewhere (pieces of lines merge in the L2: p = 2 209 ->
+  // 178 us) and with a constant velocity, where the next stage finds more of
+  // them in the caches (p = 7 75 -> 73.5 us, p = 8 86 -> 80, p = 15 91 -> 88).
+  static constexpr bool NT = !CVEL && (NQ2 % 16 == 0 || NQ > 9);
+};
+
+template <int NQ, bool CVEL, bool GU, typename VT>
+__device__ __forceinline__ void
+stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restrict__ u_,
+             const VT *__restrict__ v_, const VT *__restrict__ w_, double *out_,
+             const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
+             const double *__restrict__ D_, const double *__restrict__ ell_,
+             const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
+             const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
+             const double cb_, const double dt_, const int mode_, const int dt_geo_,
+             const int rev_, const int64_t zp_) {
+  using C = Pencil<NQ, CVEL>;
+  constexpr int NQ2 = C::NQ2, NP = C::NP, EPB = C::EPB, NFT = 6 * NQ2;
+  constexpr int S1 = C::S1, S2 = C::S2;
+  extern __shared__ double smem[];
+  const int tid = threadIdx.x;
+  const int64_t slot0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * EPB;
+  const bool lane_ok = tid < EPB * NQ2;
+  const int el = lane_ok ? tid / NQ2 : 0;
+  const int ij = lane_ok ? tid - el * NQ2 : 0;
+  const int i = ij % NQ, j = ij / NQ;
+  const int64_t slot = slot0 + el;
+  const bool active = lane_ok && slot < Ne_;
+  int64_t e;
+  if (EPB == 1) {
+    // one element per workgroup: its index, neighbour table entries and
+    // geometry record are wave-uniform and read through the scalar cache
+    e = slot < Ne_ ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
+    e = uniform(e);
+  } else {
+    e = active ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
+  }
+  const int64_t base = e * NP + ij;
+  const bool rk = mode_ == 1;
+  const bool use_q0 = rk && ca_ != 0.0;
+  constexpr bool NT_SLAB = C::NT;
+
+  // ---- loads, all in flight before anything else is asked for: with several
+  // elements per workgroup the neighbour table entries (per-lane loads) first,
+  // with one the field columns first (the entries are scalar loads, read at
+  // once); the geometry record last
+  double qc[NQ], qP[6], vP[6], q0v[NQ];
+  VT uc[NQ], vc[NQ], wc[NQ];
+  auto load_col = [&](VT (&c)[NQ], const VT *p) {
+    if constexpr (!CVEL) {
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) c[k] = p[base + (int64_t)k * NQ2];
+    }
+  };
+  auto load_q0 = [&]() {
+    if (use_q0) {
+#pragma unroll
+      for (int k = 0; k < NQ; ++k)
+        q0v[k] = NT_SLAB ? __builtin_nontemporal_load(q0_ + base + (int64_t)k * NQ2)
+                         : q0_[base + (int64_t)k * NQ2];
+    }
+  };
+  auto load_q = [&]() {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) qc[k] = q_[base + (int64_t)k * NQ2];
+    load_col(uc, u_);
+  };
+  auto load_trace = [&](int f, int64_t pidx) {
+    qP[f] = q_[pidx];
+    if constexpr (!CVEL)
+      vP[f] = (double)(kFaceAxis[f] == 0 ? u_ : kFaceAxis[f] == 1 ? v_ : w_)[pidx];
+  };
+  if (active) {
+    constexpr int order[6] = {3, 1, 0, 2, 4, 5};  // in the order of use
+    if (vmapP_) {
+      load_q();
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const int f = order[n];
+        load_trace(f, (int64_t)vmapP_[e * NFT + f * NQ2 + ij]);
+      }
+    } else {
+      int32_t nb[6];
+#pragma unroll
+      for (int f = 0; f < 6; ++f) nb[f] = nbr_[e * 6 + f];
+      load_q();
+#pragma unroll
+      for (int n = 0; n < 6; ++n) {
+        const int f = order[n];
+        load_trace(f, (int64_t)nb[f] * NP + nbr_face_node(f, i, j, NQ));
+      }
+    }
+    if constexpr (!C::LATE) {
+      load_col(vc, v_);
+      load_col(wc, w_);
+      load_q0();
+    }
+  }
+  double *const B1 = smem + el * C::SE, *const B2 = B1 + C::BUF;
+  double *const G = smem + C::OFF_G + el * 4 * NQ2, *const sL = smem + C::OFF_L;
+  for (int t = tid; t < 2 * NQ; t += C::THREADS) sL[t] = ell_[t];
+  const int zo = i + j * S1, xo = i * S1 + j * S2, yo = i + j * S2;
+  const double *g_lane = geo_ + (active && geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
+  if constexpr (EPB == 1) g_lane = geo_ + (geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
+
+  auto body = [&](const double *__restrict__ g) {
+    double cvel[3] = {0.0, 0.0, 0.0};
+    if constexpr (CVEL) {
+      cvel[0] = g[kGeoVel];
+      cvel[1] = g[kGeoVel + 1];
+      cvel[2] = g[kGeoVel + 2];
+    }
+    // flux of this lane's node of face f
+    auto face_flux = [&](int f, double qM, double vm) {
+      const double na = g[kGeoNormal + 3 * f + kFaceAxis[f]];
+      const double VelM = vm * na, VelP = (CVEL ? cvel[kFaceAxis[f]] : vP[f]) * na;
+      const double alpha = 0.5 * fabs(VelP + VelM);
+      return 0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qM * VelM - alpha * (qP[f] - qM));
+    };
+    // ---- x pencils
+    if (active) {
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        B1[zo + k * S2] = qc[k];
+        if constexpr (!CVEL) B2[zo + k * S2] = (double)uc[k];
+      }
+    }
+    __syncthreads();
+    double F[NQ], qy[NQ], acc[NQ];
+    if (active) {
+      double ux0 = cvel[0], ux1 = cvel[0], qx0, qx1;
+#pragma unroll
+      for (int l = 0; l < NQ; ++l) {
+        const double qq = B1[xo + l], uu = CVEL ? cvel[0] : B2[xo + l];
+        if (l == 0) { qx0 = qq; ux0 = uu; }
+        if (l == NQ - 1) { qx1 = qq; ux1 = uu; }
+        F[l] = qq * uu;
+      }
+#pragma unroll
+      for (int l = 0; l < NQ; ++l) qy[l] = B1[yo + l * S1];
+      G[3 * NQ2 + ij] = face_flux(3, qx0, ux0);
+      G[1 * NQ2 + ij] = face_flux(1, qx1, ux1);
+      if constexpr (C::LATE) load_col(vc, v_);
+      contract<NQ>(D_, F, acc);
+    }
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int l = 0; l < NQ; ++l) B1[xo + l] = acc[l];
+      if constexpr (!CVEL) {
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) B2[zo + k * S2] = (double)vc[k];
+      }
+    }
+    __syncthreads();
+    // ---- y pencils
+    const double Ex = g[kGeoEscale], Ey = g[kGeoEscale + 1], Ez = g[kGeoEscale + 2];
+    if (active) {
+      double vy0 = cvel[1], vy1 = cvel[1];
+#pragma unroll
+      for (int l = 0; l < NQ; ++l) {
+        const double vv = CVEL ? cvel[1] : B2[yo + l * S1];
+        if (l == 0) vy0 = vv;
+        if (l == NQ - 1) vy1 = vv;
+        F[l] = qy[l] * vv;
+      }
+      G[0 * NQ2 + ij] = face_flux(0, qy[0], vy0);
+      G[2 * NQ2 + ij] = face_flux(2, qy[NQ - 1], vy1);
+      if constexpr (C::LATE) {
+        load_col(wc, w_);
+        load_q0();
+      }
+      contract<NQ>(D_, F, acc);
+#pragma unroll
+      for (int c = 0; c < NQ; ++c) {
+        const double dx = B1[yo + c * S1];
+        B1[yo + c * S1] = combine_xy(Ex, dx, Ey, acc[c]);
+      }
+    }
+    __syncthreads();
+    // ---- z pencils
+    if (active) {
+      const double gf4 = face_flux(4, qc[0], CVEL ? cvel[2] : (double)wc[0]);
+      const double gf5 = face_flux(5, qc[NQ - 1], CVEL ? cvel[2] : (double)wc[NQ - 1]);
+#pragma unroll
+      for (int l = 0; l < NQ; ++l) F[l] = qc[l] * (CVEL ? cvel[2] : (double)wc[l]);
+      contract<NQ>(D_, F, acc);
+      const double lmi = sL[i], lpi = sL[NQ + i], lmj = sL[j], lpj = sL[NQ + j];
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        const double lift = lmj * G[0 * NQ2 + i + k * NQ] + lpi * G[1 * NQ2 + j + k * NQ] +
+                            lpj * G[2 * NQ2 + i + k * NQ] + lmi * G[3 * NQ2 + j + k * NQ] +
+                            ell_[k] * gf4 + ell_[NQ + k] * gf5;
+        const double tend = -((B1[zo + k * S2] + Ez * acc[k]) + lift);
         const int64_t idx = base + (int64_t)k * NQ2;
         double res = tend;
         if (rk) {
@@ -409,8 +689,8 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
 
 template <int NQ, bool VREG, bool AXAL, bool CVEL, bool GU>
 __global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, VREG>::THREADS),
-                               amdgpu_waves_per_eu(AXAL ? Staged<NQ, VREG>::MIN_WAVES_EU_AX
-                                                        : Staged<NQ, VREG>::MIN_WAVES_EU)))
+                               amdgpu_waves_per_eu(VREG && AXAL ? Pencil<NQ, CVEL>::MIN_WAVES_EU
+                                                                : Staged<NQ, VREG>::MIN_WAVES_EU)))
 stage_f64(const double *__restrict__ q_, const double *q0_, const double *__restrict__ u_,
           const double *__restrict__ v_, const double *__restrict__ w_, double *out_,
           const double *__restrict__ flux_in_, const int32_t *__restrict__ nbr_,
@@ -418,18 +698,22 @@ stage_f64(const double *__restrict__ q_, const double *q0_, const double *__rest
           const double *__restrict__ ell_, const double *__restrict__ geo_,
           const uint32_t *__restrict__ geoid_, const int32_t *__restrict__ order_,
           const int64_t Ne_, const double ca_, const double cb_, const double dt_,
-          const int mode_, const int axis_aligned_, const int dt_geo_, const int rev_,
+          const int mode_, const int dt_geo_, const int rev_,
           const int64_t zp_) {
-  stage_valu<NQ, VREG, AXAL, CVEL, GU, double>(q_, q0_, u_, v_, w_, out_, flux_in_, nbr_,
-                                               vmapP_, D_, ell_, geo_, geoid_, order_, Ne_,
-                                               ca_, cb_, dt_, mode_, axis_aligned_, dt_geo_,
-                                               rev_, zp_);
+  if constexpr (VREG && AXAL)
+    stage_pencil<NQ, CVEL, GU, double>(q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_,
+                                       geoid_, order_, Ne_, ca_, cb_, dt_, mode_, dt_geo_, rev_,
+                                       zp_);
+  else
+    stage_valu<NQ, VREG, AXAL, CVEL, GU, double>(q_, q0_, u_, v_, w_, out_, flux_in_, nbr_,
+                                                 vmapP_, D_, ell_, geo_, geoid_, order_, Ne_,
+                                                 ca_, cb_, dt_, mode_, dt_geo_, rev_, zp_);
 }
 
 // The mixed form's VALU kernel (register form, FP32 velocity fields).
 template <int NQ, bool AXAL, bool CVEL, bool GU>
 __global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, true>::THREADS),
-                               amdgpu_waves_per_eu(AXAL ? Staged<NQ, true>::MIN_WAVES_EU_AX
+                               amdgpu_waves_per_eu(AXAL ? Pencil<NQ, CVEL>::MIN_WAVES_EU
                                                         : Staged<NQ, true>::MIN_WAVES_EU)))
 stage_f64_mp(const double *__restrict__ q_, const double *q0_, const float *__restrict__ u_,
              const float *__restrict__ v_, const float *__restrict__ w_, double *out_,
@@ -437,11 +721,16 @@ stage_f64_mp(const double *__restrict__ q_, const double *q0_, const float *__re
              const double *__restrict__ D_, const double *__restrict__ ell_,
              const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
              const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
-             const double cb_, const double dt_, const int mode_, const int axis_aligned_,
-             const int dt_geo_, const int rev_, const int64_t zp_) {
-  stage_valu<NQ, true, AXAL, CVEL, GU, float>(q_, q0_, u_, v_, w_, out_, nullptr, nbr_, vmapP_,
-                                              D_, ell_, geo_, geoid_, order_, Ne_, ca_, cb_,
-                                              dt_, mode_, axis_aligned_, dt_geo_, rev_, zp_);
+             const double cb_, const double dt_, const int mode_, const int dt_geo_,
+             const int rev_, const int64_t zp_) {
+  if constexpr (AXAL)
+    stage_pencil<NQ, CVEL, GU, float>(q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_,
+                                      geoid_, order_, Ne_, ca_, cb_, dt_, mode_, dt_geo_, rev_,
+                                      zp_);
+  else
+    stage_valu<NQ, true, AXAL, CVEL, GU, float>(q_, q0_, u_, v_, w_, out_, nullptr, nbr_,
+                                                vmapP_, D_, ell_, geo_, geoid_, order_, Ne_,
+                                                ca_, cb_, dt_, mode_, dt_geo_, rev_, zp_);
 }
 
 // Stored-Lift kernel: Lift_mat read as stored (any Lift_mat).
@@ -579,6 +868,11 @@ stage_f64_lift(const StageArgs P) {
   }
 }
 
+template <int NQ, bool VREG, bool AXAL, bool CVEL>
+constexpr size_t valu_lds() {
+  return VREG && AXAL ? Pencil<NQ, CVEL>::LDS_BYTES : Staged<NQ, VREG>::LDS_BYTES;
+}
+
 template <int NQ, bool VREG, bool AXAL, bool CVEL, bool GU>
 int prepare_form_valu() {
   // set once per device; concurrent callers may both set it (idempotent)
@@ -588,7 +882,7 @@ int prepare_form_valu() {
   if (prepared_dev.load(std::memory_order_acquire) != dev) {
     DGK_HIP(hipFuncSetAttribute((const void *)stage_f64<NQ, VREG, AXAL, CVEL, GU>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)Staged<NQ, VREG>::LDS_BYTES));
+                                (int)valu_lds<NQ, VREG, AXAL, CVEL>()));
     prepared_dev.store(dev, std::memory_order_release);
   }
   return DGK_OK;
@@ -617,13 +911,15 @@ int prepare_nq() {
   return prepare_shape_valu<NQ, true, true>();
 }
 
-// The VALU kernels keep the element numbering where an XCD's eighth of a
-// period is under 96 elements (per launch at about 1.7e7 DOF: p = 9..13 with
-// 84..40 elements per eighth ran 1-4% slower in the XCD-interleaved order;
-// p = 2..8 with 903..98 elements 2-11% faster).  The MFMA kernels take the
-// interleaved order at every size.
+// The staged and general-normal VALU kernels keep the element numbering where
+// an XCD's eighth of a period is under 96 elements (per launch at about 1.7e7
+// DOF: p = 9..13 with 84..40 elements per eighth ran 1-4% slower in the
+// XCD-interleaved order; p = 2..8 with 903..98 elements 2-11% faster).  The
+// pencil and MFMA kernels take the interleaved order at every size (pencil,
+// with velocity fields, numbering -> order: p = 9 160 -> 153, p = 10 143 ->
+// 138, p = 12 160 -> 153, p = 15 160 -> 147 us).
 constexpr int64_t kValuMinEighth = 96;
-int64_t valu_period(int64_t q) { return q / 8 >= kValuMinEighth ? q : 0; }
+int64_t valu_period(int64_t q, bool pencil) { return pencil || q / 8 >= kValuMinEighth ? q : 0; }
 
 template <int NQ, bool VREG, bool AXAL, bool CVEL, bool GU>
 int launch_form_valu(const StageArgs &a, hipStream_t s) {
@@ -631,11 +927,12 @@ int launch_form_valu(const StageArgs &a, hipStream_t s) {
   const int64_t nblk = (a.Ne + T::EPB - 1) / T::EPB;
   if (nblk > INT32_MAX) return set_error(DGK_ERR_UNSUPPORTED, "too many elements");
   DGK_TRY((prepare_form_valu<NQ, VREG, AXAL, CVEL, GU>()));
+  constexpr size_t lds = valu_lds<NQ, VREG, AXAL, CVEL>();
   hipLaunchKernelGGL((stage_f64<NQ, VREG, AXAL, CVEL, GU>), dim3((unsigned)nblk),
-                     dim3(T::THREADS), T::LDS_BYTES, s, a.q, a.q0, a.u, a.v, a.w, a.out,
+                     dim3(T::THREADS), lds, s, a.q, a.q0, a.u, a.v, a.w, a.out,
                      a.flux_in, a.nbr, a.vmapP, a.D, a.ell, a.geo, a.geoid, a.order, a.Ne, a.ca,
-                     a.cb, a.dt, a.mode, a.axis_aligned, a.dt_geo, a.reverse,
-                     valu_period(a.zperiod));
+                     a.cb, a.dt, a.mode, a.dt_geo, a.reverse,
+                     valu_period(a.zperiod, VREG && AXAL));
   DGK_HIP(hipGetLastError());
   return DGK_OK;
 }
@@ -655,7 +952,8 @@ int launch_nq(const StageArgs &a, hipStream_t s, bool vreg) {
     const bool ax = a.axis_aligned != 0;
     if (a.cvel && ax && !a.flux_in && !a.vmapP)
       return vreg ? launch_valu<NQ, true, true, true>(a, s) : launch_valu<NQ, false, true, true>(a, s);
-    if (vreg) return ax ? launch_valu<NQ, true, true>(a, s) : launch_valu<NQ, true, false>(a, s);
+    // a given flux (cal_dqdt): the staged kernel, same bits
+    if (vreg && !a.flux_in) return ax ? launch_valu<NQ, true, true>(a, s) : launch_valu<NQ, true, false>(a, s);
     return ax ? launch_valu<NQ, false, true>(a, s) : launch_valu<NQ, false, false>(a, s);
   }
   using T = Tile<NQ>;
@@ -675,7 +973,7 @@ int prepare_form_valu_mp() {
   if (prepared_dev.load(std::memory_order_acquire) != dev) {
     DGK_HIP(hipFuncSetAttribute((const void *)stage_f64_mp<NQ, AXAL, CVEL, GU>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)Staged<NQ, true>::LDS_BYTES));
+                                (int)valu_lds<NQ, true, AXAL, CVEL>()));
     prepared_dev.store(dev, std::memory_order_release);
   }
   return DGK_OK;
@@ -695,10 +993,10 @@ int launch_form_valu_mp(const StageArgsMP &a, hipStream_t s) {
   if (nblk > INT32_MAX) return set_error(DGK_ERR_UNSUPPORTED, "too many elements");
   DGK_TRY((prepare_form_valu_mp<NQ, AXAL, CVEL, GU>()));
   hipLaunchKernelGGL((stage_f64_mp<NQ, AXAL, CVEL, GU>), dim3((unsigned)nblk),
-                     dim3(T::THREADS), T::LDS_BYTES, s, a.q, a.q0, a.u, a.v, a.w, a.out,
-                     a.nbr, a.vmapP, a.D64, a.ell64, a.geo, a.geoid, a.order, a.Ne, a.ca,
-                     a.cb, a.dt, a.mode, a.axis_aligned, a.dt_geo, a.reverse,
-                     valu_period(a.zperiod));
+                     dim3(T::THREADS), (valu_lds<NQ, true, AXAL, CVEL>()), s, a.q, a.q0, a.u,
+                     a.v, a.w, a.out, a.nbr, a.vmapP, a.D64, a.ell64, a.geo, a.geoid, a.order, a.Ne, a.ca,
+                     a.cb, a.dt, a.mode, a.dt_geo, a.reverse,
+                     valu_period(a.zperiod, AXAL));
   DGK_HIP(hipGetLastError());
   return DGK_OK;
 }
@@ -885,12 +1183,13 @@ std::atomic<int> g_f64_shape[kMaxNq + 1] = {0, 0, 0, 0, 0, 1, 0, 1, 1, 1, 1, 1, 
                                             3, 3, 1, 1, 0, 0};
 // Defaults of constant-velocity launches (batches, served requests), from the
 // same timings with the velocity read from the geometry record: the register
-// VALU kernel also at p = 2, 3 (185 -> 165 and 155 -> 140 us per launch).
+// VALU (pencil) kernel at every p <= 13 (one batched box against the staged
+// kernel: p = 1 183 -> 161, p = 3 158 -> 128, p = 5 142 -> 99 us per launch).
 // Only shapes that give the bits of the default above are taken, so a served
 // request equals its solve on a plain solver.
-constexpr int kF64DefaultCvel[kMaxNq + 1] = {0, 0, 0, 1, 1, 1, 0, 1, 1, 1, 1, 1, 1, 1, 1, 3, 3,
+constexpr int kF64DefaultCvel[kMaxNq + 1] = {0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 3, 3,
                                              1, 1, 0, 0};
-std::atomic<int> g_f64_shape_cvel[kMaxNq + 1] = {0, 0, 0, 1, 1, 1, 0, 1, 1, 1, 1, 1, 1, 1, 1,
+std::atomic<int> g_f64_shape_cvel[kMaxNq + 1] = {0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1,
                                                  3, 3, 1, 1, 0, 0};
 
 bool stage_f64_candidate_runs(int Nq, int cand, const StageArgs &a) {

@@ -266,7 +266,7 @@ stage_run(const double *__restrict__ q_, const double *q0_, const double *__rest
       const double lift = sL[j] * G[0 * NQ2 + i + k * NQ] + sL[NQ + i] * G[1 * NQ2 + j + k * NQ] +
                           sL[NQ + j] * G[2 * NQ2 + i + k * NQ] + sL[i] * G[3 * NQ2 + j + k * NQ] +
                           sL[k] * G[4 * NQ2 + i + j * NQ] + sL[NQ + k] * G[5 * NQ2 + i + j * NQ];
-      const double tend = -(((Ex * dx + Ey * dy) + Ez * dz) + lift);
+      const double tend = -((combine_xy(Ex, dx, Ey, dy) + Ez * dz) + lift);
       if (!rk) {
         res[r] = tend;
       } else {
