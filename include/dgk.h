@@ -286,9 +286,15 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * Constant-velocity launches (batch groups of constant-velocity instances,
  * served requests, solvers whose velocity fields are constant) start from
  * defaults of their own, taken only among shapes that give the bits of the
- * defaults above: FP64 the register VALU kernel also at p = 2, 3; mixed two
- * wavefronts at p = 2, 3, one at p = 5, the direction-by-direction shape at
- * p = 6, 8, 9, 11..19.
+ * defaults above: FP64 the register VALU kernel at p <= 13; mixed four
+ * wavefronts at p = 5 and the direction-by-direction shape at p = 2, 3 and
+ * 6..19.
+ * The MFMA shapes' names stand for their order of summation: most of them now
+ * add the same products in the same order on the VALU (the same bits, faster),
+ * and all at once and direction by direction then are one kernel; the MFMA
+ * itself runs direction-by-direction launches of the mixed form at p = 16, 17,
+ * and constant-velocity ones of the mixed form at p >= 16 and of FP64 at
+ * p = 16.
  * dgk_tile_select sets the process-wide choice for that form and order, for
  * both kinds of launch (-1 restores the defaults); it holds for every solver
  * that has not been autotuned; dgk_tile_selected reports the choice for

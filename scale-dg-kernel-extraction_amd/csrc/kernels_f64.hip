@@ -38,6 +38,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "contract.hpp"
 #include "dgk_internal.hpp"
 
 namespace dgk {
@@ -402,38 +403,6 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
   else body(g_lane);
 }
 
-// acc[c] = sum over l (ascending) of D(c, l) F[l], D read through the scalar
-// cache one column ahead.  The address of column l + 1 is made opaque at a
-// point that follows column l - 1's arithmetic: otherwise the compiler loads
-// all NQ columns first, and the 2 NQ^2 scalar registers spill.
-typedef const double __attribute__((address_space(4))) *uniform_ptr;
-template <int NQ>
-__device__ __forceinline__ void contract(const double *D, const double (&F)[NQ],
-                                         double (&acc)[NQ]) {
-  uniform_ptr p = (uniform_ptr)D;
-  double cur[NQ], nxt[NQ];
-#pragma unroll
-  for (int c = 0; c < NQ; ++c) {
-    acc[c] = 0.0;
-    cur[c] = p[c];
-  }
-#pragma unroll
-  for (int l = 0; l < NQ; ++l) {
-    if (l + 1 < NQ) {
-      asm volatile("" : "+s"(p));
-#pragma unroll
-      for (int c = 0; c < NQ; ++c) asm volatile("" : "+v"(acc[c]));
-#pragma unroll
-      for (int c = 0; c < NQ; ++c) nxt[c] = p[c + (l + 1) * NQ];
-    }
-#pragma unroll
-    for (int c = 0; c < NQ; ++c) {
-      acc[c] += cur[c] * F[l];
-      cur[c] = nxt[c];
-    }
-  }
-}
-
 // Pencil form of the stage (axis-aligned faces, flux computed here): lane (a,b)
 // of an element owns in turn the x pencil (:,a,b), the y pencil (a,:,b) and the
 // z pencil (a,b,:).
@@ -443,7 +412,7 @@ __device__ __forceinline__ void contract(const double *D, const double (&F)[NQ],
 //   2. it reads the x pencils of q and u and the y pencil of q.  Face node (a,b)
 //      of the x faces is an end of the x pencil, so the upwind fluxes need no
 //      other own trace; D applies to the pencil in registers, its entries scalar
-//      operands (contract below).  Dx goes back to LDS in place of q, v in place
+//      operands (contract.hpp).  Dx goes back to LDS in place of q, v in place
 //      of u;
 //   3. the same along y; Ex Dx + Ey Dy replaces Dx;
 //   4. the same along z, Lift, RK update.
@@ -621,7 +590,7 @@ stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restr
       G[3 * NQ2 + ij] = face_flux(3, qx0, ux0);
       G[1 * NQ2 + ij] = face_flux(1, qx1, ux1);
       if constexpr (C::LATE) load_col(vc, v_);
-      contract<NQ>(D_, F, acc);
+      Contract<double, NQ, RowsAscending<NQ>>().run(D_, ell_, F, acc);
     }
     __syncthreads();
     if (active) {
@@ -650,7 +619,7 @@ stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restr
         load_col(wc, w_);
         load_q0();
       }
-      contract<NQ>(D_, F, acc);
+      Contract<double, NQ, RowsAscending<NQ>>().run(D_, ell_, F, acc);
 #pragma unroll
       for (int c = 0; c < NQ; ++c) {
         const double dx = B1[yo + c * S1];
@@ -664,27 +633,41 @@ stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restr
       const double gf5 = face_flux(5, qc[NQ - 1], CVEL ? cvel[2] : (double)wc[NQ - 1]);
 #pragma unroll
       for (int l = 0; l < NQ; ++l) F[l] = qc[l] * (CVEL ? cvel[2] : (double)wc[l]);
-      contract<NQ>(D_, F, acc);
+      Contract<double, NQ, RowsAscending<NQ>>().run(D_, ell_, F, acc);
       const double lmi = sL[i], lpi = sL[NQ + i], lmj = sL[j], lpj = sL[NQ + j];
+      const typename Contract<double, NQ, RowsAscending<NQ>>::uniform_ptr ell =
+          (typename Contract<double, NQ, RowsAscending<NQ>>::uniform_ptr)ell_;
 #pragma unroll
       for (int k = 0; k < NQ; ++k) {
         const double lift = lmj * G[0 * NQ2 + i + k * NQ] + lpi * G[1 * NQ2 + j + k * NQ] +
                             lpj * G[2 * NQ2 + i + k * NQ] + lmi * G[3 * NQ2 + j + k * NQ] +
-                            ell_[k] * gf4 + ell_[NQ + k] * gf5;
-        const double tend = -((B1[zo + k * S2] + Ez * acc[k]) + lift);
-        const int64_t idx = base + (int64_t)k * NQ2;
-        double res = tend;
-        if (rk) {
-          const double upd = cb_ * (qc[k] + (dt_geo_ ? g[kGeoDt] : dt_) * tend);
-          res = use_q0 ? ca_ * q0v[k] + upd : upd;
+                            ell[k] * gf4 + ell[NQ + k] * gf5;
+        acc[k] = -((B1[zo + k * S2] + Ez * acc[k]) + lift);
+      }
+      if (rk) {
+        const double dtv = dt_geo_ ? g[kGeoDt] : dt_;
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+          const double upd = cb_ * (qc[k] + dtv * acc[k]);
+          acc[k] = use_q0 ? ca_ * q0v[k] + upd : upd;
         }
-        if constexpr (NT_SLAB) __builtin_nontemporal_store(res, out_ + idx);
-        else out_[idx] = res;
+      }
+#pragma unroll
+      for (int k = 0; k < NQ; ++k) {
+        if constexpr (NT_SLAB) __builtin_nontemporal_store(acc[k], out_ + base + (int64_t)k * NQ2);
+        else out_[base + (int64_t)k * NQ2] = acc[k];
       }
     }
   };
-  if constexpr (GU) body(geo_);
-  else body(g_lane);
+  if constexpr (GU) {
+    body(geo_);
+  } else if constexpr (EPB > 1) {
+    const double *gb = block_record(slot0, EPB, Ne_, geo_, geoid_, order_, rev_, zp_, dt_geo_);
+    if (gb) body(gb);
+    else body(g_lane);
+  } else {
+    body(g_lane);
+  }
 }
 
 template <int NQ, bool VREG, bool AXAL, bool CVEL, bool GU>

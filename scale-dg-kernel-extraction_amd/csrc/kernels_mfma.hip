@@ -1,617 +1,11 @@
-// MFMA stage kernels (gfx950), one template for two precisions:
-//  * mixed (HIP_MP): the 1D-operator contractions and the Lift run in FP32 on
-//    v_mfma_f32_16x16x4f32 with FP32 accumulation; the state q, the face-flux
-//    jumps, the volume fluxes q*u_d and the RK stage combination stay FP64;
-//    velocities are read from FP32 copies;
-//  * FP64 (HIP, tile candidates): the same data flow in FP64 throughout, on
-//    v_mfma_f64_16x16x4f64.
-//
-// For each direction d the sum-factorised derivative and that direction's two
-// Lift faces form one GEMM over the block's "pencils" r (node lines along d):
-//   out_d(r, c) = sum_l E_d F_d(r, l) D(c, l)
-//               + l-(c) flux(face d-, r) + l+(c) flux(face d+, r)
-// i.e. A_d = [E_d F_d | flux_d- | flux_d+ | 0]  (pencils x KPAD, the zeros
-//            supplied by the operand read),
-//      B   = [D^T ; l- ; l+ ; 0]               (KPAD x NQ), the same for
-// every direction and element.  The reference's face-node order (Fmask,
-// mod_mesh.f90:278-324) is the pencil order of the face's normal direction,
-// so the Lift (tensorprod_Lift_hexahedral, mod_dg_optr_kernel.f90:262-288, in
-// its tensor-product form) is two extra K columns of the contraction
-// (tensorprod_divlike_dirXYZ, mod_dg_optr_kernel.f90:197-258).
-//
-// Data flow of one block (EPB elements, one lane per node column (i,j)):
-//   1. the lane loads its q column (FP64), its velocity columns, the own
-//      traces of the x/y faces and the neighbour traces straight into
-//      registers (coalesced along (i,j));
-//   2. FP64 upwind fluxes and FP64 volume fluxes E_d q u_d, each rounded once
-//      to the operand precision, are written into augmented A arrays in LDS,
-//      one pencil per row of an odd number of values (bank conflicts were 64%
-//      of the LDS cycles of the p = 7 mixed and p = 15 FP64 kernels, 79% at
-//      p = 18, with rows of KPAD values);
-//   3. MFMA over 16-pencil tiles; K is permuted so that lane (col, kq) keeps
-//      rows l = kq*KSTEPS + ks of B in registers and reads A at fixed offsets
-//      from its own base; the result overwrites the tile's rows in place;
-//   4. the three direction results are summed in FP64, dqdt = -((X + Y) + Z),
-//      and RK-combined in FP64 (main.f90:69-73).
-// The direction-sequential variant (SEQ) runs steps 2-3 one direction at a
-// time through one LDS area, loading each velocity column only when its
-// direction comes up: a third of the LDS and fewer live registers, for large
-// orders; it adds the directions in the same order, so its results are the
-// same bits.
-#include <algorithm>
-#include <atomic>
-
-#include "dgk_internal.hpp"
+// The mixed-precision form (HIP_MP): its instantiations of the stage kernels
+// of stage_aug.hpp, the mixed kernel over runs of consecutive elements, and the
+// selection of a tile shape per order.
+#include "stage_aug.hpp"
 
 namespace dgk {
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-// Operand precision of the contraction GEMMs.
-// Both MFMAs take A(row = lane%16, k = lane/16) and B(k = lane/16,
-// col = lane%16); result value t of a lane lies in column lane%16 and row
-// RSTRIDE_Q*(lane/16) + RSTRIDE_T*t (checked on the device for both).
-struct PrecMixed {
-  using vel_t = float;   // velocity copies read by the kernel
-  using op_t = float;    // A, B operands in LDS / registers
-  using acc_t = f32x4;   // 16x16 result, 4 values per lane
-  static constexpr int RSTRIDE_Q = 4, RSTRIDE_T = 1;
-  static __device__ __forceinline__ acc_t mfma(op_t a, op_t b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-};
-struct PrecF64 {
-  using vel_t = double;
-  using op_t = double;
-  using acc_t = f64x4;
-  static constexpr int RSTRIDE_Q = 1, RSTRIDE_T = 4;
-  static __device__ __forceinline__ acc_t mfma(op_t a, op_t b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-};
-
-__device__ __forceinline__ int xcd_block_mp(int b, int n) {
-  const int per = n >> 3, rem = n & 7;
-  const int x = b & 7, local = b >> 3;
-  return x * per + min(x, rem) + local;
-}
-
-__device__ __forceinline__ int64_t uniform_mp(int64_t v) {
-  const int lo = __builtin_amdgcn_readfirstlane((int)(v & 0xffffffff));
-  const int hi = __builtin_amdgcn_readfirstlane((int)(v >> 32));
-  return (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
-}
-
-// Tile shape of the MFMA stage kernel: EPB elements per block, all three
-// directions at once or one after the other (SEQ).
-template <class P, int NQ, int EPB_, bool SEQ_>
-struct MP {
-  static constexpr int NQ2 = NQ * NQ;
-  static constexpr int NP = NQ2 * NQ;
-  static constexpr int EPB = EPB_;
-  static constexpr bool SEQ = SEQ_;
-  static constexpr int LANES = EPB * NQ2;                   // node columns per block
-  // Above p = 15 (289..400 columns) the block is eight wavefronts, two per
-  // SIMD, the idle lanes taking GEMM tiles, and held to 4 waves per SIMD, so
-  // two blocks share a CU (per launch at about 1.7e7 DOF, p = 16..19, against
-  // 5..7 wavefronts and no cap: FP64 314/276/308/349 -> 278/270/263/320 us,
-  // mixed 171/153/180/209 -> 151/166/176/193 us)
-  static constexpr bool HI = SEQ && NQ > 16;
-  static constexpr int THREADS = HI ? 512 : ((LANES + 63) / 64) * 64;
-  static constexpr int WAVES = THREADS / 64;
-  static constexpr int ROWS = ((LANES + 15) / 16) * 16;     // pencils per direction
-  static constexpr int MTILES = ROWS / 16;
-  static constexpr int NT = (NQ + 15) / 16;                // 16-wide column tiles of B
-  static constexpr int KAUG = NQ + 2;
-  static constexpr int KSTEPS = (KAUG + 3) / 4;
-  static constexpr int KPAD = 4 * KSTEPS;
-  static constexpr int NAREA = SEQ ? 1 : 3;
-  // Operands per row of A in LDS: KAUG rounded up to odd, so that the lanes
-  // that write and read A at a stride of one row (the y and z pencils, the
-  // flux columns, the 16 rows of an MFMA operand read) spread over the banks.
-  // The K padding is not stored: the operand read puts zeros there.  KAUG
-  // itself for FP32 at p = 7, 15, where a stride of 2 (mod 8) lets the operand
-  // reads (K ranges of 3 and 5) fall into other banks too (a count of bank
-  // cycles per workgroup gives 384 and 2624 against 444 and 3056; 560 and 3776
-  // with rows of KPAD), and where the odd stride would not fit in a CU's LDS
-  // (FP64 p = 17).
-  static constexpr size_t area_bytes(int stride) {
-    return ((size_t)NAREA * ROWS * stride + 4) * sizeof(typename P::op_t);  // + read overrun
-  }
-  static constexpr bool EVEN_STRIDE = sizeof(typename P::op_t) == 4 && NQ % 8 == 0;
-  static constexpr int STRIDE =
-      !EVEN_STRIDE && area_bytes(KAUG | 1) <= 160 * 1024 ? (KAUG | 1) : KAUG;
-  static constexpr int AREA = ROWS * STRIDE;                // operands per direction
-  static constexpr size_t A_BYTES = (area_bytes(STRIDE) + 7) / 8 * 8;
-  // One-wavefront all-at-once shapes first pass the q, u, v columns through
-  // LDS, where each lane picks up its own x/y face traces (same area as A,
-  // used before it); the others load those traces from global memory (the
-  // exchange would cost them registers and a wave per SIMD)
-  static constexpr bool XCH = !SEQ && WAVES == 1;
-  // k-slabs of the exchange buffers: a slab apart by one (q, u) or eight (v)
-  // more than the lanes, so the reads of different k fall into other banks
-  static constexpr int XLS = LANES + 1, XLV = LANES + 8;
-  static constexpr size_t XCH_BYTES =
-      XCH ? (size_t)NQ * (XLS * (sizeof(double) + sizeof(typename P::vel_t)) +
-                          XLV * sizeof(typename P::vel_t))
-          : 0;
-  // Multi-wavefront all-at-once shapes up to p = 9: the face lanes put the
-  // x/y face traces into a buffer after the A area, and the x/y fluxes are
-  // formed after the barrier that already precedes the GEMMs (one barrier
-  // more; above p = 9 it cost more than the global trace loads it saves)
-  static constexpr bool XD = !SEQ && WAVES > 1 && NQ <= 10;
-  static constexpr size_t XD_BYTES =
-      XD ? (size_t)EPB * 4 * NQ2 * (sizeof(double) + sizeof(typename P::vel_t)) : 0;
-  static constexpr size_t LDS_BYTES = (A_BYTES > XCH_BYTES ? A_BYTES : XCH_BYTES) + XD_BYTES;
-  // Register budget: the mixed exchange shapes keep 4 waves per SIMD (at most
-  // 128 registers; left free, p = 7 lands two above and drops to 3), and so
-  // do the shapes above p = 15 (FP64 spills 12..60 bytes per lane)
-  static constexpr int MIN_WAVES_EU = ((sizeof(typename P::op_t) == 4 && XCH) || HI) ? 4 : 1;
-  // Shapes whose face-normal form is tested at run time (see stage_mfma).
-  static constexpr bool AX_RUNTIME = SEQ || MIN_WAVES_EU > 1;
-  static constexpr int JOBS = NAREA * MTILES;               // (direction, tile) GEMMs per pass
-  static constexpr int JPW = (JOBS + WAVES - 1) / WAVES;
-};
-
-// Candidate kinds per order: for Nq^2 <= 64 one, two or four wavefronts of
-// whole elements, then one wavefront direction by direction; above, one
-// element, two elements, and one element direction by direction; above
-// p = 15 one element, all at once or direction by direction.  Kinds whose
-// LDS exceeds a CU's 160 KiB are dropped (all at once above p = 15: FP64 up
-// to p = 17, mixed up to p = 19); the remaining ones are the candidates 0,
-// 1, ... (per-order defaults in kMpDefault below).
-constexpr int kKinds = 4;
-template <int NQ>
-constexpr int kind_epb(int k) {
-  constexpr int NQ2 = NQ * NQ;
-  if (NQ2 <= 64) {
-    const int waves = k == 1 ? 2 : k == 2 ? 4 : 1;
-    const int e = 64 * waves / NQ2;
-    return e < 1 ? 1 : e;
-  }
-  return k == 1 ? 2 : 1;
-}
-template <int NQ>
-constexpr bool kind_seq(int k) {
-  return NQ * NQ > 64 ? k == 2 : k == 3;
-}
-template <class P, int NQ>
-constexpr bool kind_ok(int k) {
-  if (NQ * NQ > 64 && k == 3) return false;
-  if (NQ > kMaxNqValu && k == 1) return false;  // above p = 15: one element per workgroup
-  return k == 0   ? MP<P, NQ, kind_epb<NQ>(0), kind_seq<NQ>(0)>::LDS_BYTES <= 160 * 1024
-         : k == 1 ? MP<P, NQ, kind_epb<NQ>(1), kind_seq<NQ>(1)>::LDS_BYTES <= 160 * 1024
-         : k == 2 ? MP<P, NQ, kind_epb<NQ>(2), kind_seq<NQ>(2)>::LDS_BYTES <= 160 * 1024
-                  : MP<P, NQ, kind_epb<NQ>(3), kind_seq<NQ>(3)>::LDS_BYTES <= 160 * 1024;
-}
-template <class P, int NQ>
-constexpr int ncand() {
-  return (int)kind_ok<P, NQ>(0) + (int)kind_ok<P, NQ>(1) + (int)kind_ok<P, NQ>(2) +
-         (int)kind_ok<P, NQ>(3);
-}
-// kind of candidate c (-1 if none)
-template <class P, int NQ>
-constexpr int kind_of(int c) {
-  int n = 0;
-  for (int k = 0; k < kKinds; ++k) {
-    if (!kind_ok<P, NQ>(k)) continue;
-    if (n == c) return k;
-    ++n;
-  }
-  return -1;
-}
-
-// One 16-pencil tile: A rows (STRIDE operands apart) from `tile`, B (NT column
-// tiles) in registers; all A values are read before any result overwrites the
-// tile's first NQ columns.  `left` = KAUG - kq * KSTEPS: operands of this
-// lane's K range from there on are padding, read as whatever follows the row
-// and replaced by zero.
-template <class P, int KSTEPS, int KAUG, int STRIDE, int NQ, int NT>
-__device__ __forceinline__ void mfma_tile(typename P::op_t *tile,
-                                          const typename P::op_t (&bop)[NT][KSTEPS], int rd,
-                                          int wr, int col, int left) {
-  typename P::op_t a[KSTEPS];
-#pragma unroll
-  for (int ks = 0; ks < KSTEPS; ++ks) {
-    const typename P::op_t v = tile[rd + ks];
-    a[ks] = 3 * KSTEPS + ks < KAUG || ks < left ? v : (typename P::op_t)0;
-  }
-  typename P::acc_t acc[NT];
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    acc[nt] = typename P::acc_t{0, 0, 0, 0};
-#pragma unroll
-    for (int ks = 0; ks < KSTEPS; ++ks) acc[nt] = P::mfma(a[ks], bop[nt][ks], acc[nt]);
-  }
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    if (16 * nt + col < NQ) {
-#pragma unroll
-      for (int t4 = 0; t4 < 4; ++t4) tile[wr + 16 * nt + t4 * P::RSTRIDE_T * STRIDE] = acc[nt][t4];
-    }
-  }
-}
-
-// AXAL: every face normal lies along its face's axis (checked on the host); a
-// compile-time form, so the axis-aligned kernel holds no registers for the
-// general normal velocity (one more wave per SIMD for several multi-wavefront
-// shapes, e.g. the mixed p = 10, 11, 15 defaults).  Two kinds of shape keep
-// the test at run time (AX_RUNTIME), because decided at compile time their
-// allocations grow: the direction-by-direction (SEQ) shapes (p = 5..9:
-// 5 -> 4 waves per SIMD) and the mixed one-wavefront shapes held to 4 waves
-// (p = 2..4 then spill 2 to 24 VGPRs).
-// CVEL: constant velocity per element, (u, v, w) = words kGeoVel..+2 of its
-// geometry record (batched and served boxes); no velocity field is read, and
-// the operand-precision value of a constant is the value its per-node copy
-// holds, so the results are the same bits.
-// GU: several elements per workgroup and one geometry record for the whole
-// launch (no per-element record ids): the record is read through the kernel
-// argument itself, i.e. through the scalar cache (as in stage_f64).
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL = false, bool GU = false>
-__global__ void __attribute__((amdgpu_flat_work_group_size(1, MP<P, NQ, EPB, SEQ>::THREADS),
-                               amdgpu_waves_per_eu(MP<P, NQ, EPB, SEQ>::MIN_WAVES_EU)))
-stage_mfma(const double *__restrict__ q_, const double *q0_,
-           const typename P::vel_t *__restrict__ u_, const typename P::vel_t *__restrict__ v_,
-           const typename P::vel_t *__restrict__ w_, double *out_,
-           const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
-           const typename P::op_t *__restrict__ D_, const typename P::op_t *__restrict__ ell_,
-           const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
-           const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
-           const double cb_, const double dt_, const int mode_, const int axis_aligned_,
-           const int dt_geo_, const int rev_, const int64_t zp_) {
-  using C = MP<P, NQ, EPB, SEQ>;
-  using vel_t = typename P::vel_t;
-  using op_t = typename P::op_t;
-  constexpr int NQ2 = C::NQ2, NP = C::NP, NFT = 6 * NQ2, KSTEPS = C::KSTEPS;
-  constexpr int KAUG = C::KAUG, STRIDE = C::STRIDE;
-  constexpr int AREA = C::AREA;
-  extern __shared__ double smem_mp[];
-  op_t *const As = (op_t *)smem_mp;
-
-  const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63;
-  const int64_t slot0 = (int64_t)xcd_block_mp(blockIdx.x, gridDim.x) * EPB;
-  const bool lane_ok = tid < C::LANES;
-  const int el = lane_ok ? tid / NQ2 : 0;
-  const int ij = lane_ok ? tid - el * NQ2 : 0;
-  const int i = ij % NQ, j = ij / NQ;
-  const int64_t slot = slot0 + el;
-  const bool active = lane_ok && slot < Ne_;
-  int64_t e;
-  const double *g_lane;
-  if (EPB == 1) {
-    e = slot < Ne_ ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
-    e = uniform_mp(e);
-    g_lane = geo_ + (geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
-  } else {
-    e = active ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
-    g_lane = geo_ + (active && geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
-  }
-  static_assert(!GU || EPB > 1, "one element per workgroup reads its record uniformly anyway");
-  auto body = [&](const double *__restrict__ g) {
-    const int64_t ebase = e * NP;
-    const int64_t base = ebase + ij;
-    const bool rk = mode_ == 1;
-    const bool use_q0 = rk && ca_ != 0.0;
-    const bool axal = C::AX_RUNTIME ? axis_aligned_ != 0 : AXAL;
-    const int R = el * NQ2;
-    const vel_t *const velp[3] = {u_, v_, w_};
-    vel_t cv[3] = {(vel_t)0, (vel_t)0, (vel_t)0};
-    if constexpr (CVEL) {
-      cv[0] = (vel_t)g[kGeoVel];
-      cv[1] = (vel_t)g[kGeoVel + 1];
-      cv[2] = (vel_t)g[kGeoVel + 2];
-    }
-
-    // ---- 1. loads straight into registers ------------------------------------
-    // Neighbour-table entries: with several elements per workgroup they are
-    // per-lane loads, issued first so that waiting for them before the trace
-    // gathers does not also wait for the column loads behind them; with one
-    // they are scalar loads read where used (fewer live registers at high
-    // order).
-    int32_t nb6[6] = {};
-    const bool resolved = vmapP_ != nullptr;
-    if constexpr (EPB > 1) {
-      if (active) nbr_entries<NQ>(vmapP_, nbr_, e, ij, nb6);
-    }
-    auto nbr_at = [&](int f) -> int64_t {
-      if constexpr (EPB > 1) return nbr_node<NQ>(resolved, nb6[f], f, i, j);
-      return resolved ? (int64_t)vmapP_[e * NFT + f * NQ2 + ij]
-                      : (int64_t)nbr_[e * 6 + f] * NP + nbr_face_node(f, i, j, NQ);
-    };
-    double qc[NQ];
-    vel_t uc[SEQ ? 1 : NQ], vc[SEQ ? 1 : NQ], wc[NQ];  // SEQ: w only at k = 0, NQ-1
-    double qM[4], qP[6];
-    vel_t vM[4], vP[6];  // velocity component along the face axis
-    if (active) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        qc[k] = q_[base + k * NQ2];
-        if constexpr (!SEQ) {
-          uc[k] = CVEL ? cv[0] : u_[base + k * NQ2];
-          vc[k] = CVEL ? cv[1] : v_[base + k * NQ2];
-          wc[k] = CVEL ? cv[2] : w_[base + k * NQ2];
-        }
-      }
-      if constexpr (SEQ) {
-        wc[0] = CVEL ? cv[2] : w_[base];
-        wc[NQ - 1] = CVEL ? cv[2] : w_[base + (NQ - 1) * NQ2];
-      }
-      if constexpr (!C::XCH && !C::XD) {
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {  // own traces of the x and y faces
-          const int64_t m = ebase + own_face_node(f, i, j, NQ);
-          qM[f] = q_[m];
-          vM[f] = CVEL ? cv[kFaceAxis[f]] : (kFaceAxis[f] == 0 ? u_ : v_)[m];
-        }
-      }
-#pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int64_t pidx = nbr_at(f);
-        qP[f] = q_[pidx];
-        vP[f] = CVEL ? cv[kFaceAxis[f]]
-                     : (kFaceAxis[f] == 0 ? u_ : kFaceAxis[f] == 1 ? v_ : w_)[pidx];
-      }
-    }
-
-    // ---- 1b. own x/y face traces from the lanes that hold them (XCH) --------
-    // Face node (a,b) of face f lies in the column of lane (a,0), (NQ-1,a),
-    // (a,NQ-1) or (0,a) at k = b; every lane stores its q, u, v columns in LDS
-    // and reads its four traces back, with no global loads (they would be
-    // gathers of one cache line per two lanes on the x faces).
-    if constexpr (C::XCH) {
-      double *xq = (double *)smem_mp;
-      vel_t *xu = (vel_t *)(xq + C::XLS * NQ), *xv = xu + C::XLS * NQ;
-      if (active) {
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-          xq[k * C::XLS + tid] = qc[k];
-          if constexpr (!CVEL) {
-            xu[k * C::XLS + tid] = uc[k];
-            xv[k * C::XLV + tid] = vc[k];
-          }
-        }
-      }
-      __syncthreads();
-      if (active) {
-        const int src[4] = {R + i, R + (NQ - 1) + i * NQ, R + i + (NQ - 1) * NQ, R + i * NQ};
-#pragma unroll
-        for (int f = 0; f < 4; ++f) {
-          qM[f] = xq[j * C::XLS + src[f]];
-          vM[f] = CVEL                  ? cv[kFaceAxis[f]]
-                  : kFaceAxis[f] == 0 ? xu[j * C::XLS + src[f]]
-                                      : xv[j * C::XLV + src[f]];
-        }
-      }
-      __syncthreads();  // the A operands below reuse the area
-    }
-
-    double *xd_q = (double *)((char *)smem_mp + C::A_BYTES) + el * 4 * NQ2;
-    vel_t *xd_v =
-        (vel_t *)((double *)((char *)smem_mp + C::A_BYTES) + EPB * 4 * NQ2) + el * 4 * NQ2;
-    if constexpr (C::XD) {
-      if (active) {
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-          if (j == 0) {
-            xd_q[0 * NQ2 + i + k * NQ] = qc[k];
-            xd_v[0 * NQ2 + i + k * NQ] = vc[k];
-          }
-          if (i == NQ - 1) {
-            xd_q[1 * NQ2 + j + k * NQ] = qc[k];
-            xd_v[1 * NQ2 + j + k * NQ] = uc[k];
-          }
-          if (j == NQ - 1) {
-            xd_q[2 * NQ2 + i + k * NQ] = qc[k];
-            xd_v[2 * NQ2 + i + k * NQ] = vc[k];
-          }
-          if (i == 0) {
-            xd_q[3 * NQ2 + j + k * NQ] = qc[k];
-            xd_v[3 * NQ2 + j + k * NQ] = uc[k];
-          }
-        }
-      }
-    }
-    // ---- 2a. FP64 upwind fluxes -------------------------------------------------
-    op_t fl[6];
-    auto face_flux = [&](int f) {
-      {
-        const double qm = f == 4 ? qc[0] : f == 5 ? qc[NQ - 1] : qM[f];
-        double VelM, VelP;
-        if (axal) {
-          const int ax = kFaceAxis[f];
-          const double na = g[kGeoNormal + 3 * f + ax];
-          const vel_t vm = f == 4 ? wc[0] : f == 5 ? wc[NQ - 1] : vM[f];
-          VelM = (double)vm * na;
-          VelP = (double)vP[f] * na;
-        } else {
-          // general normals: all three components on both sides
-          const int64_t m = ebase + own_face_node(f, i, j, NQ);
-          const int64_t pidx = nbr_at(f);
-          const double n1 = g[kGeoNormal + 3 * f], n2 = g[kGeoNormal + 3 * f + 1],
-                       n3 = g[kGeoNormal + 3 * f + 2];
-          if constexpr (CVEL) {
-            VelM = (double)cv[0] * n1 + (double)cv[1] * n2 + (double)cv[2] * n3;
-            VelP = VelM;
-            (void)m;
-            (void)pidx;
-          } else {
-            VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
-            VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
-          }
-        }
-        const double alpha = 0.5 * fabs(VelP + VelM);
-        fl[f] = (op_t)(0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qm * VelM - alpha * (qP[f] - qm)));
-      }
-    };
-    if (active) {
-#pragma unroll
-      for (int f = C::XD ? 4 : 0; f < 6; ++f) face_flux(f);
-    }
-
-    // B = [D^T ; l- ; l+ ; 0] rows of this lane (k permuted, see above)
-    constexpr int NT = C::NT;
-    const int col = lane & 15, kq = lane >> 4;
-    op_t bop[NT][KSTEPS];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int c = 16 * nt + col;
-#pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int l = kq * KSTEPS + ks;
-        bop[nt][ks] = c >= NQ ? (op_t)0 : l < NQ ? D_[c + l * NQ] : l == NQ ? ell_[c]
-                      : l == NQ + 1 ? ell_[NQ + c] : (op_t)0;
-      }
-    }
-    const int rd = col * STRIDE + kq * KSTEPS;        // A read offset of this lane in a tile
-    const int wr = P::RSTRIDE_Q * kq * STRIDE + col;  // result offset of value 0
-    const int left = KAUG - kq * KSTEPS;              // stored operands of the lane's K range
-    // Node (i,j,k) sits in the x pencil (j,k) at position i, in the y pencil
-    // (i,k) at position j and in the z pencil (i,j) at position k; face node
-    // (i,j) of the faces normal to d is pencil ij of direction d.
-    const int pos_off[3] = {(R + j) * STRIDE + i, (R + i) * STRIDE + j, (R + ij) * STRIDE};
-    const int pos_step[3] = {NQ * STRIDE, NQ * STRIDE, 1};
-    // non-temporal RK base and output where k-slabs are whole 128-byte lines;
-    // cached where one instruction covers pieces of lines (p <= 6), so the L2
-    // merges them (as stage_f64; mixed p = 2, 4: 6% faster per launch)
-    constexpr bool NT_SLAB = (NQ2 % 16 == 0) || NQ > 7;
-    const int face_m[3] = {3, 0, 4}, face_p[3] = {1, 2, 5};  // -d and +d faces
-
-    double q0v[NQ];
-    double tend[NQ];
-    if constexpr (!SEQ) {
-      // ---- 2b. volume fluxes of all three directions -> A arrays ------------
-      if (active) {
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          const double Ed = g[kGeoEscale + d];
-          op_t *a = As + d * AREA + pos_off[d];
-#pragma unroll
-          for (int k = 0; k < NQ; ++k) {
-            const vel_t vel = d == 0 ? uc[k] : d == 1 ? vc[k] : wc[k];
-            a[k * pos_step[d]] = (op_t)(Ed * (qc[k] * (double)vel));
-          }
-          op_t *r = As + d * AREA + (R + ij) * STRIDE;
-          if (!C::XD || d == 2) {
-            r[NQ] = fl[face_m[d]];
-            r[NQ + 1] = fl[face_p[d]];
-          }
-        }
-      }
-      // RK base column, in flight during the GEMMs (the RK base and the output
-      // are touched once per launch: non-temporal, so L2 keeps the neighbour
-      // traces)
-      if (active && use_q0) {
-#pragma unroll
-        for (int k = 0; k < NQ; ++k)
-          q0v[k] = NT_SLAB ? __builtin_nontemporal_load(q0_ + base + k * NQ2) : q0_[base + k * NQ2];
-      }
-      __syncthreads();
-      if constexpr (C::XD) {
-        if (active) {
-#pragma unroll
-          for (int f = 0; f < 4; ++f) {
-            qM[f] = xd_q[f * NQ2 + ij];
-            vM[f] = CVEL ? cv[kFaceAxis[f]] : xd_v[f * NQ2 + ij];
-            face_flux(f);
-          }
-#pragma unroll
-          for (int d = 0; d < 2; ++d) {
-            op_t *r = As + d * AREA + (R + ij) * STRIDE;
-            r[NQ] = fl[face_m[d]];
-            r[NQ + 1] = fl[face_p[d]];
-          }
-        }
-        __syncthreads();
-      }
-
-      // ---- 3. MFMA GEMMs over (direction, 16-pencil tile) jobs ---------------
-      // Rows of A beyond the block's active pencils hold stale LDS; each output
-      // row depends only on its own A row, and those rows are never read back.
-#pragma unroll
-      for (int jj = 0; jj < C::JPW; ++jj) {
-        const int job = wave + jj * C::WAVES;
-        if (job >= C::JOBS) break;  // wave-uniform
-        const int d = job / C::MTILES, t = job - d * C::MTILES;
-        mfma_tile<P, KSTEPS, KAUG, STRIDE, NQ, NT>(As + d * AREA + t * 16 * STRIDE, bop, rd, wr,
-                                                   col, left);
-      }
-      __syncthreads();
-
-      // ---- 4a. FP64 sum of the three directions ------------------------------
-      if (active) {
-#pragma unroll
-        for (int k = 0; k < NQ; ++k)
-          tend[k] = ((double)As[pos_off[0] + k * pos_step[0]] +
-                     (double)As[AREA + pos_off[1] + k * pos_step[1]]) +
-                    (double)As[2 * AREA + pos_off[2] + k * pos_step[2]];
-      }
-    } else {
-      // ---- 2b-4a, one direction at a time through one LDS area ---------------
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        if (active) {
-          const double Ed = g[kGeoEscale + d];
-          const vel_t *vel = velp[d];
-          op_t *a = As + pos_off[d];
-#pragma unroll
-          for (int k = 0; k < NQ; ++k)
-            a[k * pos_step[d]] =
-                (op_t)(Ed * (qc[k] * (double)(CVEL ? cv[d] : vel[base + k * NQ2])));
-          op_t *r = As + (R + ij) * STRIDE;
-          r[NQ] = fl[face_m[d]];
-          r[NQ + 1] = fl[face_p[d]];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int jj = 0; jj < C::JPW; ++jj) {
-          const int t = wave + jj * C::WAVES;
-          if (t >= C::MTILES) break;  // wave-uniform
-          mfma_tile<P, KSTEPS, KAUG, STRIDE, NQ, NT>(As + t * 16 * STRIDE, bop, rd, wr, col, left);
-        }
-        __syncthreads();
-        if (active) {
-#pragma unroll
-          for (int k = 0; k < NQ; ++k) {
-            const double x = (double)As[pos_off[d] + k * pos_step[d]];
-            tend[k] = d == 0 ? x : tend[k] + x;
-          }
-        }
-        if (d < 2) __syncthreads();  // the next direction overwrites the area
-      }
-    }
-
-    // ---- 4b. RK epilogue (FP64) -------------------------------------------------
-    // SEQ reads the RK base only here: held through the last direction's GEMM it
-    // cost p = 16, 17 a wave per SIMD (FP64 Nq = 17: 154 -> 124 VGPRs; p = 16
-    // 399 -> 313 us per launch, p = 17 344 -> 276, mixed p = 19 271 -> 208)
-    if (SEQ && active && use_q0) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k)
-        q0v[k] = NT_SLAB ? __builtin_nontemporal_load(q0_ + base + k * NQ2) : q0_[base + k * NQ2];
-    }
-    if (active) {
-      const double dtv = dt_geo_ ? g[kGeoDt] : dt_;
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        const double td = -tend[k];
-        const int64_t idx = base + (int64_t)k * NQ2;
-        double res = td;
-        if (rk) {
-          const double upd = cb_ * (qc[k] + dtv * td);
-          res = use_q0 ? ca_ * q0v[k] + upd : upd;
-        }
-        if constexpr (NT_SLAB) __builtin_nontemporal_store(res, out_ + idx);
-        else out_[idx] = res;
-      }
-    }
-  };
-  if constexpr (GU) body(geo_);
-  else body(g_lane);
-}
 
 // ---- mixed precision over runs of consecutive elements (p <= 4) -----------
 // stage_run_mp<NQ, AXAL>: the data flow of the FP64 run kernel
@@ -941,81 +335,6 @@ int launch_run_mp(int Nq, const StageArgsMP &a, hipStream_t s) {
   }
 }
 
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL, bool GU>
-int prepare_kernel() {
-  // set once per device; concurrent callers may both set it (idempotent)
-  static std::atomic<int> prepared_dev{-1};
-  int dev = 0;
-  DGK_HIP(hipGetDevice(&dev));
-  if (prepared_dev.load(std::memory_order_acquire) != dev) {
-    DGK_HIP(hipFuncSetAttribute((const void *)stage_mfma<P, NQ, EPB, SEQ, AXAL, CVEL, GU>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)MP<P, NQ, EPB, SEQ>::LDS_BYTES));
-    prepared_dev.store(dev, std::memory_order_release);
-  }
-  return DGK_OK;
-}
-
-// a form with its uniform-geometry variant where a workgroup holds several
-// elements
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL = false>
-int prepare_form() {
-  DGK_TRY((prepare_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, false>()));
-  if constexpr (EPB > 1) DGK_TRY((prepare_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, true>()));
-  return DGK_OK;
-}
-
-// Both face-normal forms of a shape (one, testing at run time, for the
-// AX_RUNTIME shapes).
-template <class P, int NQ, int EPB, bool SEQ>
-int prepare_shape() {
-  constexpr bool AXR = MP<P, NQ, EPB, SEQ>::AX_RUNTIME;
-  DGK_TRY((prepare_form<P, NQ, EPB, SEQ, false>()));
-  if constexpr (!AXR) DGK_TRY((prepare_form<P, NQ, EPB, SEQ, true>()));
-  DGK_TRY((prepare_form<P, NQ, EPB, SEQ, !AXR, true>()));
-  return DGK_OK;
-}
-
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL, bool GU, class Args>
-int launch_kernel(const Args &a, hipStream_t s) {
-  using T = MP<P, NQ, EPB, SEQ>;
-  const int64_t nblk = (a.Ne + T::EPB - 1) / T::EPB;
-  if (nblk > INT32_MAX) return set_error(DGK_ERR_UNSUPPORTED, "too many elements");
-  DGK_TRY((prepare_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, GU>()));
-  hipLaunchKernelGGL((stage_mfma<P, NQ, EPB, SEQ, AXAL, CVEL, GU>), dim3((unsigned)nblk),
-                     dim3(T::THREADS), T::LDS_BYTES, s, a.q, a.q0, a.u, a.v, a.w, a.out, a.nbr,
-                     a.vmapP, a.D, a.ell, a.geo, a.geoid, a.order, a.Ne, a.ca, a.cb, a.dt,
-                     a.mode, a.axis_aligned, a.dt_geo, a.reverse, a.zperiod);
-  DGK_HIP(hipGetLastError());
-  return DGK_OK;
-}
-
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, class Args, bool CVEL = false>
-int launch_form(const Args &a, hipStream_t s) {
-  if constexpr (EPB > 1)
-    if (!a.geoid) return launch_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, true>(a, s);
-  return launch_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, false>(a, s);
-}
-
-template <class P, int NQ, int EPB, bool SEQ, class Args>
-int launch_shape(const Args &a, hipStream_t s) {
-  constexpr bool AXR = MP<P, NQ, EPB, SEQ>::AX_RUNTIME;
-  // constant velocity: batched and served boxes, whose faces are axis-aligned
-  if (a.cvel && a.axis_aligned && !a.vmapP)
-    return launch_form<P, NQ, EPB, SEQ, !AXR, Args, true>(a, s);
-  if constexpr (!AXR)
-    if (a.axis_aligned) return launch_form<P, NQ, EPB, SEQ, true>(a, s);
-  return launch_form<P, NQ, EPB, SEQ, false>(a, s);
-}
-
-// Candidate c of order NQ (compile-time), as a kernel instantiation.
-template <class P, int NQ, int CAND>
-struct Cand {
-  static constexpr int K = kind_of<P, NQ>(CAND);
-  static constexpr int EPB = kind_epb<NQ>(K < 0 ? 0 : K);
-  static constexpr bool SEQ = kind_seq<NQ>(K < 0 ? 0 : K);
-};
-
 // Tile-shape candidate selected per Nq for the mixed form.  Defaults from
 // per-order timings on MI355X at about 1.7e7 DOF (whole-step runs, every
 // candidate, with a launch-wide geometry record read through the scalar
@@ -1031,67 +350,20 @@ constexpr int kMpDefault[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
                                         0, 0, 0, 0, 2, 0, 1, 1, 0, 0};
 std::atomic<int> g_mp_shape[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
                                            0, 0, 0, 0, 2, 0, 1, 1, 0, 0};
-// Defaults of constant-velocity launches (batches, served requests), from the
-// same timings with the velocity read from the geometry record, among the
-// shapes that give the bits of the default above (the MFMA shapes and the
-// run kernel), so a served request equals its solve on a plain solver: two
-// wavefronts at p = 2, 3 (183 -> 161 and 150 -> 148 us per launch against
-// one), one wavefront at p = 5 (129 -> 108 us against two), and direction by
-// direction at p = 6, 8, 9, 11..19 where it needs a third of the LDS and no
-// velocity load sits between its directions (p = 8 105 -> 98, p = 12 101 ->
-// 99, p = 13 94 -> 89, p = 15 97 -> 90, p = 18 131 -> 110, p = 19 137 ->
-// 119 us).
-constexpr int kMpDefaultCvel[kMaxNq + 1] = {0, 0, 5, 1, 1, 1, 0, 3, 0, 2, 2,
-                                            0, 2, 2, 2, 2, 2, 1, 1, 1, 1};
-std::atomic<int> g_mp_shape_cvel[kMaxNq + 1] = {0, 0, 5, 1, 1, 1, 0, 3, 0, 2, 2,
-                                                0, 2, 2, 2, 2, 2, 1, 1, 1, 1};
-
-template <class P, int NQ>
-int prepare_nq_all() {
-  DGK_TRY((prepare_shape<P, NQ, Cand<P, NQ, 0>::EPB, Cand<P, NQ, 0>::SEQ>()));
-  if constexpr (ncand<P, NQ>() > 1)
-    DGK_TRY((prepare_shape<P, NQ, Cand<P, NQ, 1>::EPB, Cand<P, NQ, 1>::SEQ>()));
-  if constexpr (ncand<P, NQ>() > 2)
-    DGK_TRY((prepare_shape<P, NQ, Cand<P, NQ, 2>::EPB, Cand<P, NQ, 2>::SEQ>()));
-  if constexpr (ncand<P, NQ>() > 3)
-    DGK_TRY((prepare_shape<P, NQ, Cand<P, NQ, 3>::EPB, Cand<P, NQ, 3>::SEQ>()));
-  return DGK_OK;
-}
-
-template <class P, int NQ, class Args>
-int launch_nq_cand(int cand, const Args &a, hipStream_t s) {
-  if constexpr (ncand<P, NQ>() > 1)
-    if (cand == 1) return launch_shape<P, NQ, Cand<P, NQ, 1>::EPB, Cand<P, NQ, 1>::SEQ>(a, s);
-  if constexpr (ncand<P, NQ>() > 2)
-    if (cand == 2) return launch_shape<P, NQ, Cand<P, NQ, 2>::EPB, Cand<P, NQ, 2>::SEQ>(a, s);
-  if constexpr (ncand<P, NQ>() > 3)
-    if (cand == 3) return launch_shape<P, NQ, Cand<P, NQ, 3>::EPB, Cand<P, NQ, 3>::SEQ>(a, s);
-  return launch_shape<P, NQ, Cand<P, NQ, 0>::EPB, Cand<P, NQ, 0>::SEQ>(a, s);
-}
-
-template <class P, int NQ>
-int shapes_of(int *epb) {
-  constexpr int n = ncand<P, NQ>();
-  if constexpr (n > 0) epb[0] = Cand<P, NQ, 0>::EPB;
-  if constexpr (n > 1) epb[1] = Cand<P, NQ, 1>::EPB;
-  if constexpr (n > 2) epb[2] = Cand<P, NQ, 2>::EPB;
-  if constexpr (n > 3) epb[3] = Cand<P, NQ, 3>::EPB;
-  return n;
-}
+// Defaults of constant-velocity launches (batches, served requests, solvers with
+// constant fields), from the same timings with the velocity read from the
+// geometry record, among the shapes that give the bits of the default above
+// (all but the VALU kernel), so a served request equals its solve on a plain
+// solver: two wavefronts at p = 4 (59 against 64 us per launch with one), four
+// at p = 5 (75 against 85 on a solver, 84 against 89 on a batched box), one
+// (direction by direction: the same kernel) else; above p = 15 direction by
+// direction, on the MFMA.
+constexpr int kMpDefaultCvel[kMaxNq + 1] = {0, 0, 5, 3, 3, 1, 2, 3, 3, 2, 2,
+                                            2, 2, 2, 2, 2, 2, 1, 1, 1, 1};
+std::atomic<int> g_mp_shape_cvel[kMaxNq + 1] = {0, 0, 5, 3, 3, 1, 2, 3, 3, 2, 2,
+                                                2, 2, 2, 2, 2, 2, 1, 1, 1, 1};
 
 }  // namespace
-
-#define DGK_NQ_SWITCH(NQV, CALL)                                                         \
-  switch (NQV) {                                                                         \
-  case 2: return CALL(2); case 3: return CALL(3); case 4: return CALL(4);                \
-  case 5: return CALL(5); case 6: return CALL(6); case 7: return CALL(7);                \
-  case 8: return CALL(8); case 9: return CALL(9); case 10: return CALL(10);              \
-  case 11: return CALL(11); case 12: return CALL(12); case 13: return CALL(13);          \
-  case 14: return CALL(14); case 15: return CALL(15); case 16: return CALL(16);          \
-  case 17: return CALL(17); case 18: return CALL(18); case 19: return CALL(19);          \
-  case 20: return CALL(20);                                                              \
-  default: return set_error(DGK_ERR_UNSUPPORTED, "Nq outside 2.." + std::to_string(kMaxNq));                   \
-  }
 
 static int mp_mfma_shapes(int Nq, int *epb);
 
@@ -1140,19 +412,6 @@ int launch_stage_mp(int Nq, const StageArgsMP &a, hipStream_t s) {
 #undef DGK_CALL
 }
 
-int prepare_tile_f64(int Nq) {
-#define DGK_CALL(N) prepare_nq_all<PrecF64, N>()
-  DGK_NQ_SWITCH(Nq, DGK_CALL)
-#undef DGK_CALL
-}
-
-int launch_tile_f64(int Nq, int cand, const StageArgs &a, hipStream_t s) {
-  if (a.Ne < 1) return DGK_OK;
-#define DGK_CALL(N) launch_nq_cand<PrecF64, N>(cand, a, s)
-  DGK_NQ_SWITCH(Nq, DGK_CALL)
-#undef DGK_CALL
-}
-
 static int mp_mfma_shapes(int Nq, int *epb) {
 #define DGK_CALL(N) shapes_of<PrecMixed, N>(epb)
   DGK_NQ_SWITCH(Nq, DGK_CALL)
@@ -1165,13 +424,6 @@ int stage_mp_shapes(int Nq, int *epb, int n) {
   if (nc > 0 && run_mp_elements(Nq) > 0) epb[nc++] = run_mp_elements(Nq);
   if (nc > 0 && valu_mp_elements(Nq) > 0) epb[nc++] = valu_mp_elements(Nq);
   return nc;
-}
-
-int tile_f64_shapes(int Nq, int *epb, int n) {
-  if (Nq < kMinNq || Nq > kMaxNq || !epb || n < kKinds) return 0;
-#define DGK_CALL(N) shapes_of<PrecF64, N>(epb)
-  DGK_NQ_SWITCH(Nq, DGK_CALL)
-#undef DGK_CALL
 }
 
 int stage_mp_select(int Nq, int cand) {
@@ -1192,7 +444,5 @@ int stage_mp_selected(int Nq) {
 int stage_mp_selected_cvel(int Nq) {
   return (Nq < kMinNq || Nq > kMaxNq) ? 0 : g_mp_shape_cvel[Nq].load(std::memory_order_relaxed);
 }
-
-#undef DGK_NQ_SWITCH
 
 }  // namespace dgk
