@@ -288,6 +288,7 @@ int create_from_tables(int evaltype, MeshTables &t, dgk_solver **out) {
   const bool use_ell = sep_dev <= kSeparableF64;
 
   auto *s = new dgk_solver();
+  transfer_retain();
   auto fail = [&](int rc) {
     dgk_destroy(s);
     return rc;
@@ -473,6 +474,7 @@ int dgk_destroy(dgk_solver *s) {
   for (hipEvent_t e : s->free_events) (void)hipEventDestroy(e);
   for (void *p : s->allocs) (void)hipFree(p);
   if (s->stream) (void)hipStreamDestroy(s->stream);
+  transfer_release();
   delete s;
   return DGK_OK;
 }
@@ -546,7 +548,7 @@ int dgk_get_field(dgk_solver *s, int which, double *f, int64_t n) {
   if (n != owned && !with_halo) return set_error(DGK_ERR_ARG, "field length must be Np*Ne or Np*NeA");
   if (which == DGK_FIELD_DQDT && !s->dqdt) return set_error(DGK_ERR_STATE, "dqdt has not been computed");
   const double *src = field_ptr(s, which);
-  DGK_HIP(hipMemcpyAsync(f, src, sizeof(double) * owned, hipMemcpyDeviceToHost, s->stream));
+  DGK_TRY(download(f, src, (int64_t)sizeof(double) * owned, s->device, s->stream));
   if (with_halo) {
     const int64_t tail = (int64_t)s->Np * s->NeA - owned;
     if (which == DGK_FIELD_DQDT) {
@@ -592,9 +594,7 @@ int dgk_cal_elembnd_flux(dgk_solver *s, double *flux_host) {
   tm.done();
   s->flux_valid = true;
   if (flux_host) {
-    DGK_HIP(hipMemcpyAsync(flux_host, s->flux, sizeof(double) * n, hipMemcpyDeviceToHost,
-                           s->stream));
-    DGK_HIP(hipStreamSynchronize(s->stream));
+    DGK_TRY(download(flux_host, s->flux, (int64_t)sizeof(double) * n, s->device, s->stream));
   }
   return DGK_OK;
 }
@@ -633,9 +633,7 @@ int dgk_cal_tend(dgk_solver *s, double *dqdt_host) {
   tm.done();
   s->dqdt_valid = true;
   if (dqdt_host) {
-    DGK_HIP(hipMemcpyAsync(dqdt_host, s->dqdt, sizeof(double) * n, hipMemcpyDeviceToHost,
-                           s->stream));
-    DGK_HIP(hipStreamSynchronize(s->stream));
+    DGK_TRY(download(dqdt_host, s->dqdt, (int64_t)sizeof(double) * n, s->device, s->stream));
   }
   return DGK_OK;
 }
@@ -1085,10 +1083,8 @@ int dgk_batch_get_field(dgk_batch *b, int inst, int which, double *f, int64_t n)
   const int64_t off = l->elem_off * s->Np, cnt = l->Ne * s->Np;
   if (n != cnt) return set_error(DGK_ERR_ARG, "field length must be Np*Ne of the instance");
   DGK_HIP(hipStreamSynchronize(b->stream));
-  DGK_HIP(hipMemcpyAsync(f, field_ptr(s, which) + off, sizeof(double) * cnt,
-                         hipMemcpyDeviceToHost, s->stream));
-  DGK_HIP(hipStreamSynchronize(s->stream));
-  return DGK_OK;
+  return download(f, field_ptr(s, which) + off, (int64_t)sizeof(double) * cnt, s->device,
+                  s->stream);
 }
 
 int dgk_batch_init_gaussian(dgk_batch *b, int inst, double cx, double cy, double cz,

@@ -453,9 +453,8 @@ int retire(dgk_server *sv, Req *r) {
   res.mass = slot[2];
   res.l2sq = slot[3];
   if (r->r.q_out) {
-    DGK_HIP(hipMemcpyAsync(r->r.q_out, r->s.q[0], sizeof(double) * r->dof,
-                           hipMemcpyDeviceToHost, sv->copy_stream));
-    DGK_HIP(hipStreamSynchronize(sv->copy_stream));
+    DGK_TRY(download(r->r.q_out, r->s.q[0], (int64_t)sizeof(double) * r->dof, sv->device,
+                     sv->copy_stream));
   }
   res.t_done = seconds_since(sv->t0);
   sv->arena.release(r->off, r->bytes);
@@ -624,11 +623,13 @@ int dgk_serve_create(const char *operator_dir, int64_t hbm_budget, int max_activ
     return set_error(DGK_ERR_DEVICE, "no HIP device available (the path has no CPU fallback)");
   }
   auto *sv = new dgk_server();
+  transfer_retain();
   auto fail = [&](int rc) {
     for (hipStream_t s : sv->streams) (void)hipStreamDestroy(s);
     if (sv->copy_stream) (void)hipStreamDestroy(sv->copy_stream);
     if (sv->arena.base) (void)hipFree(sv->arena.base);
     if (sv->pinned) (void)hipHostFree(sv->pinned);
+    transfer_release();
     delete sv;
     return rc;
   };
@@ -785,6 +786,7 @@ int dgk_serve_destroy(dgk_server *sv) {
   }
   if (sv->arena.base) (void)hipFree(sv->arena.base);
   if (sv->pinned) (void)hipHostFree(sv->pinned);
+  transfer_release();
   delete sv;
   return DGK_OK;
 }

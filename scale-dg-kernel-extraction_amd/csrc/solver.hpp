@@ -94,6 +94,12 @@ int upload(dgk_solver *s, T *dst, const std::vector<T> &src) {
 }
 
 double *field_ptr(dgk_solver *s, int which);
+// Copy `bytes` from the device to the caller's host memory after everything
+// enqueued on `s`, and wait for it (transfer.cpp).  Handles that download hold
+// a reference to the shared staging memory while they live.
+int download(void *dst, const void *src, int64_t bytes, int device, hipStream_t s);
+void transfer_retain();
+void transfer_release();
 int refresh_f32(dgk_solver *s, int which);
 // One stage launch on `stream` (the solver's own stream when nullptr);
 // dt_geo takes the time step from each element's geometry record.
