@@ -36,7 +36,8 @@ hipEvent_t take_event(dgk_solver *s) {
     return e;
   }
   hipEvent_t e = nullptr;
-  if (hipEventCreate(&e) != hipSuccess) return nullptr;
+  // timing only: without the fence to system scope that a default event brings
+  if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) return nullptr;
   return e;
 }
 
@@ -351,6 +352,8 @@ int create_from_tables(int evaltype, MeshTables &t, dgk_solver **out) {
         break;
       }
   }
+  if (hipMemsetAsync(s->mm + 2 * kMinmaxBlocks, 0, sizeof(double), s->stream) != hipSuccess)
+    return fail(set_error(DGK_ERR_DEVICE, "hipMemsetAsync failed"));
   for (int b = 0; b < 3; ++b)
     if (hipMemsetAsync(s->q[b], 0, sizeof(double) * s->nfield, s->stream) != hipSuccess)
       return fail(set_error(DGK_ERR_DEVICE, "hipMemsetAsync failed"));
@@ -473,6 +476,7 @@ int dgk_destroy(dgk_solver *s) {
   }
   for (hipEvent_t e : s->free_events) (void)hipEventDestroy(e);
   for (void *p : s->allocs) (void)hipFree(p);
+  if (s->mm_host) (void)hipHostFree(s->mm_host);
   if (s->stream) (void)hipStreamDestroy(s->stream);
   transfer_release();
   delete s;
@@ -680,14 +684,18 @@ int dgk_minmax(dgk_solver *s, double *qmin, double *qmax) {
   DGK_TRY(enter(s));
   if (!s->set[DGK_FIELD_Q]) return set_error(DGK_ERR_STATE, "q not set");
   const int64_t n = (int64_t)s->Np * s->Ne;
-  DGK_TRY(launch_minmax(s->q[s->cur], n, s->mm, kMinmaxBlocks, s->mm + 2 * kMinmaxBlocks,
-                        s->stream));
-  double r[2];
-  DGK_HIP(hipMemcpyAsync(r, s->mm + 2 * kMinmaxBlocks, sizeof(r), hipMemcpyDeviceToHost,
-                         s->stream));
+  if (!s->mm_host) {
+    if (hipHostMalloc((void **)&s->mm_host, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      s->mm_host = nullptr;
+      return set_error(DGK_ERR_NOMEM, "hipHostMalloc of the min/max result failed");
+    }
+  }
+  DGK_TRY(launch_minmax_once(s->q[s->cur], n, s->mm, (uint32_t *)(s->mm + 2 * kMinmaxBlocks),
+                             s->mm_host, s->stream));
   DGK_HIP(hipStreamSynchronize(s->stream));
-  if (qmin) *qmin = r[0];
-  if (qmax) *qmax = r[1];
+  if (qmin) *qmin = s->mm_host[0];
+  if (qmax) *qmax = s->mm_host[1];
   return resolve_timers(s);  // the stream is idle: folding costs no wait
 }
 

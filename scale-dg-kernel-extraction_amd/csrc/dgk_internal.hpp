@@ -348,8 +348,10 @@ int launch_halo_gather(double *f, const int32_t *src, int64_t base,
                        int64_t n, hipStream_t s);
 int launch_rk_update(double *q, const double *q0, const double *dqdt,
                      double a, double b, double dt, int64_t n, hipStream_t s);
-int launch_minmax(const double *q, int64_t n, double *partial, int nblk,
-                  double *result, hipStream_t s);
+// min/max of n doubles into result[0..1], device or mapped host memory;
+// partial: 2 kMinmaxBlocks doubles, *counter zero before and after.
+int launch_minmax_once(const double *q, int64_t n, double *partial, uint32_t *counter,
+                       double *result, hipStream_t s);
 int launch_to_f32(const double *src, float *dst, int64_t n, hipStream_t s);
 // *flag = 1 if some f[t] differs (bit for bit) from f[0], else 0.
 int launch_varies(const double *f, int64_t n, int32_t *flag, hipStream_t s);

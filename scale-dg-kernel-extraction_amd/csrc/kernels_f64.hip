@@ -1084,6 +1084,62 @@ __global__ void minmax_final(const double *partial, int nblk, double *result) {
   }
 }
 
+// min/max of q in one launch, into host memory: the block that finishes last
+// folds the others' partials, writes the pair through the mapped pointer and
+// leaves the counter at zero for the next launch.  At the small sizes where a
+// host looks at every step, a second launch and a copy of 16 bytes cost more
+// than the reduction (8^3 elements at p = 3: 26 -> 16 us with the wait).
+__device__ __forceinline__ void block_minmax(double &mn, double &mx) {
+  __shared__ double smin[4], smax[4];
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    mn = fmin(mn, __shfl_xor(mn, d));
+    mx = fmax(mx, __shfl_xor(mx, d));
+  }
+  __syncthreads();  // the buffers may still be read from a call before
+  if ((threadIdx.x & 63) == 0) {
+    smin[threadIdx.x >> 6] = mn;
+    smax[threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  mn = fmin(fmin(smin[0], smin[1]), fmin(smin[2], smin[3]));
+  mx = fmax(fmax(smax[0], smax[1]), fmax(smax[2], smax[3]));
+}
+__global__ void __launch_bounds__(256)
+minmax_once(const double *__restrict__ q, int64_t n, double *partial, uint32_t *counter,
+            double *result) {
+  __shared__ bool last;
+  double mn = INFINITY, mx = -INFINITY;
+  for (int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x; t < n; t += (int64_t)gridDim.x * 256) {
+    const double x = q[t];
+    mn = fmin(mn, x);
+    mx = fmax(mx, x);
+  }
+  block_minmax(mn, mx);
+  if (threadIdx.x == 0) {
+    __hip_atomic_store(partial + 2 * blockIdx.x, mn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(partial + 2 * blockIdx.x + 1, mx, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+    last = __hip_atomic_fetch_add(counter, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+           gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return;
+  mn = INFINITY;
+  mx = -INFINITY;
+  for (int t = threadIdx.x; t < (int)gridDim.x; t += 256) {
+    mn = fmin(mn, __hip_atomic_load(partial + 2 * t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    mx = fmax(mx,
+              __hip_atomic_load(partial + 2 * t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  }
+  block_minmax(mn, mx);
+  if (threadIdx.x == 0) {
+    result[0] = mn;
+    result[1] = mx;
+    *counter = 0;
+  }
+}
+
 // Periodic Gaussian blob exp(-r^2/(2 sigma^2)) (minimum-image distance) and
 // constant velocity on a NeX x NeY x NeZ box, node coordinates as in
 // set_element_position (mod_mesh.f90:332-353).
@@ -1339,8 +1395,21 @@ int launch_rk_update(double *q, const double *q0, const double *dqdt, double a,
   return DGK_OK;
 }
 
-int launch_minmax(const double *q, int64_t n, double *partial, int nblk,
-                  double *result, hipStream_t s) {
+// blocks of a min/max over n values: one per 2048, strided over beyond `most`
+static int minmax_blocks(int64_t n, int most) {
+  return (int)std::min<int64_t>(most, std::max<int64_t>(1, (n + 2047) / 2048));
+}
+
+int launch_minmax_once(const double *q, int64_t n, double *partial, uint32_t *counter,
+                       double *result, hipStream_t s) {
+  hipLaunchKernelGGL(minmax_once, dim3(minmax_blocks(n, kMinmaxBlocks)), dim3(256), 0, s, q, n,
+                     partial, counter, result);
+  DGK_HIP(hipGetLastError());
+  return DGK_OK;
+}
+
+static int launch_minmax(const double *q, int64_t n, double *partial, int nblk,
+                         double *result, hipStream_t s) {
   hipLaunchKernelGGL(minmax_partial, dim3(nblk), dim3(256), 0, s, q, n, partial);
   DGK_HIP(hipGetLastError());
   hipLaunchKernelGGL(minmax_final, dim3(1), dim3(256), 0, s, partial, nblk, result);
@@ -1384,10 +1453,7 @@ static int scratch_address(double **out) {
 int launch_minmax_noalloc(const double *q, int64_t n, double *result, hipStream_t s) {
   double *partial = nullptr;
   DGK_TRY(scratch_address(&partial));
-  // one block per 2048 values, at most kNoallocBlocks; blocks stride over the rest
-  const int64_t want = (n + 2047) / 2048;
-  const int nblk = (int)std::min<int64_t>(kNoallocBlocks, std::max<int64_t>(1, want));
-  return launch_minmax(q, n, partial, nblk, result, s);
+  return launch_minmax(q, n, partial, minmax_blocks(n, kNoallocBlocks), result, s);
 }
 
 int launch_init_gaussian(double *q, double *u, double *v, double *w, const double *x1D,

@@ -53,7 +53,8 @@ struct dgk_solver {
   int32_t *nbr = nullptr, *vmapP = nullptr, *halo = nullptr;
   double *geo = nullptr, *D = nullptr, *Lift = nullptr;
   uint32_t *geoid = nullptr;
-  double *mm = nullptr;  // min/max partials + result
+  double *mm = nullptr;       // min/max partials, then the block counter
+  double *mm_host = nullptr;  // pinned: min, max (made by the first dgk_minmax)
   bool set[4] = {false, false, false, false};
   int64_t bytes = 0;
   std::vector<void *> allocs;
