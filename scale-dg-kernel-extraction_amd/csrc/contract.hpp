@@ -28,7 +28,7 @@ struct RowsAscending {
 // opaque addresses and the ties on acc it loads all of B first and spills it.
 template <class T, int NQ, class Rows>
 struct Contract {
-    static constexpr int W = 128 / (int)sizeof(T);
+  static constexpr int W = 128 / (int)sizeof(T);
   static constexpr int TOTAL = Rows::N * NQ;
   static constexpr int BATCHES = (TOTAL + W - 1) / W;
   typedef const T __attribute__((address_space(4))) *uniform_ptr;

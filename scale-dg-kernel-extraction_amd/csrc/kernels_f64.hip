@@ -421,7 +421,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
 // contractions one operand at a time (LDS busy 52% of the cycles), and the
 // scalar loads before its first field load.  This one makes 124 (108 with a
 // constant velocity, and half the LDS).  us per launch at about 1.7e7 DOF,
-// start -> now, velocity fields: p = 4 168 -> 159, p = 7 142 -> 129, p = 8
+// before -> now, velocity fields: p = 4 168 -> 159, p = 7 142 -> 129, p = 8
 // 163 -> 146, p = 11 159 -> 138, p = 12 187 -> 153, p = 13 181 -> 161; a
 // solver's constant velocity (it read the fields): p = 1 187 -> 102, p = 3
 // 154 -> 77, p = 7 142 -> 74 (4.8 TB/s), p = 12 187 -> 90.  What is left with
