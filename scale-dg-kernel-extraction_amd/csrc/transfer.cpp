@@ -98,6 +98,18 @@ hipError_t copy_slice(const Pool &p, int l, char *dst, const char *src, int64_t 
   return e;
 }
 
+// Ordinary pageable memory, the only kind the slices are for: the runtime
+// copies straight into pinned memory at the link's rate, and a thread cannot
+// write device memory.
+bool pageable(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
 }  // namespace
 
 void transfer_retain() {
@@ -111,7 +123,7 @@ void transfer_release() {
 }
 
 int download(void *dst, const void *src, int64_t bytes, int device, hipStream_t s) {
-  if (bytes >= kSliced) {
+  if (bytes >= kSliced && pageable(dst)) {
     std::unique_lock<std::mutex> lk(g_pool.mu, std::try_to_lock);
     // another download has the pool, it is not made yet, or it belongs to
     // another device: plain copy
