@@ -619,6 +619,11 @@ int dgk_cal_dqdt(dgk_solver *s, const double *flux_host) {
   if (!s->dqdt) DGK_TRY(dalloc(s, &s->dqdt, (int64_t)s->Np * s->Ne));
   StageArgs a = stage_args(s, s->q[s->cur], nullptr, s->dqdt, 0, 0.0, 1.0, 0.0);
   a.flux_in = s->flux;
+  // these launches read the velocity fields, whatever the solver's stages do
+  if (a.cvel) {
+    a.cvel = 0;
+    a.tile = s->tile_other;
+  }
   Timed tm(s, T_DQDT, s->kernel_timing);
   DGK_TRY(launch_stage_f64(s->Nq, a, s->stream));
   tm.done();

@@ -95,6 +95,9 @@ struct Staged {
   // register form at p = 11, which otherwise lands one VGPR above the
   // 168 that 3 waves allow (and drops to 2).
   static constexpr int MIN_WAVES_EU = (VREG && NQ == 12) ? 3 : 1;
+  // The given-flux kernel: 5 waves at p = 4 (108 VGPRs -> 96 or fewer; 153 ->
+  // 147 us per launch) and 3 at p = 13 (186 -> 168 with 6 spilled; 196 -> 172).
+  static constexpr int MIN_WAVES_EU_FLUX = NQ == 14 ? 3 : NQ == 5 ? 5 : 1;
 };
 
 // AXAL: every face normal lies along its face's axis (checked on the host), so
@@ -693,6 +696,27 @@ stage_f64(const double *__restrict__ q_, const double *q0_, const double *__rest
                                                  ca_, cb_, dt_, mode_, dt_geo_, rev_, zp_);
 }
 
+// A given face flux (cal_dqdt) in the register form.  No trace and no normal is
+// read, so one kernel serves both normal forms; with the pointer known not to be
+// null their code and registers go.  us per launch at about 1.7e7 DOF, staged
+// form against this one: p = 4 163/150, p = 7 176/141, p = 11 203/158, p = 12
+// 243/191, p = 13 293/172.
+template <int NQ, bool GU>
+__global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, true>::THREADS),
+                               amdgpu_waves_per_eu(Staged<NQ, true>::MIN_WAVES_EU_FLUX)))
+stage_f64_flux(const double *__restrict__ q_, const double *q0_, const double *__restrict__ u_,
+               const double *__restrict__ v_, const double *__restrict__ w_, double *out_,
+               const double *__restrict__ flux_in_, const double *__restrict__ D_,
+               const double *__restrict__ ell_, const double *__restrict__ geo_,
+               const uint32_t *__restrict__ geoid_, const int32_t *__restrict__ order_,
+               const int64_t Ne_, const double ca_, const double cb_, const double dt_,
+               const int mode_, const int dt_geo_, const int rev_, const int64_t zp_) {
+  if (!flux_in_) __builtin_unreachable();
+  stage_valu<NQ, true, false, false, GU, double>(q_, q0_, u_, v_, w_, out_, flux_in_, nullptr,
+                                                 nullptr, D_, ell_, geo_, geoid_, order_, Ne_,
+                                                 ca_, cb_, dt_, mode_, dt_geo_, rev_, zp_);
+}
+
 // The mixed form's VALU kernel (register form, FP32 velocity fields).
 template <int NQ, bool AXAL, bool CVEL, bool GU>
 __global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, true>::THREADS),
@@ -884,6 +908,20 @@ int prepare_shape_valu() {
   return DGK_OK;
 }
 
+template <int NQ, bool GU>
+int prepare_flux() {
+  static std::atomic<int> prepared_dev{-1};
+  int dev = 0;
+  DGK_HIP(hipGetDevice(&dev));
+  if (prepared_dev.load(std::memory_order_acquire) != dev) {
+    DGK_HIP(hipFuncSetAttribute((const void *)stage_f64_flux<NQ, GU>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)Staged<NQ, true>::LDS_BYTES));
+    prepared_dev.store(dev, std::memory_order_release);
+  }
+  return DGK_OK;
+}
+
 template <int NQ>
 int prepare_nq() {
   DGK_TRY((prepare_shape_valu<NQ, false, false>()));
@@ -891,6 +929,8 @@ int prepare_nq() {
   DGK_TRY((prepare_shape_valu<NQ, true, false>()));
   DGK_TRY((prepare_shape_valu<NQ, false, true, true>()));
   DGK_TRY((prepare_shape_valu<NQ, true, true, true>()));
+  DGK_TRY((prepare_flux<NQ, false>()));
+  if constexpr (has_gu<NQ, true>()) DGK_TRY((prepare_flux<NQ, true>()));
   return prepare_shape_valu<NQ, true, true>();
 }
 
@@ -927,6 +967,20 @@ int launch_valu(const StageArgs &a, hipStream_t s) {
   return launch_form_valu<NQ, VREG, AXAL, CVEL, false>(a, s);
 }
 
+template <int NQ, bool GU>
+int launch_flux(const StageArgs &a, hipStream_t s) {
+  using T = Staged<NQ, true>;
+  const int64_t nblk = (a.Ne + T::EPB - 1) / T::EPB;
+  if (nblk > INT32_MAX) return set_error(DGK_ERR_UNSUPPORTED, "too many elements");
+  DGK_TRY((prepare_flux<NQ, GU>()));
+  hipLaunchKernelGGL((stage_f64_flux<NQ, GU>), dim3((unsigned)nblk), dim3(T::THREADS),
+                     T::LDS_BYTES, s, a.q, a.q0, a.u, a.v, a.w, a.out, a.flux_in, a.D, a.ell,
+                     a.geo, a.geoid, a.order, a.Ne, a.ca, a.cb, a.dt, a.mode, a.dt_geo,
+                     a.reverse, valu_period(a.zperiod, false));
+  DGK_HIP(hipGetLastError());
+  return DGK_OK;
+}
+
 // VALU stage kernel (VREG: v, w in registers; the axis-aligned or general
 // normal form), or the stored-Lift kernel.
 template <int NQ>
@@ -935,8 +989,12 @@ int launch_nq(const StageArgs &a, hipStream_t s, bool vreg) {
     const bool ax = a.axis_aligned != 0;
     if (a.cvel && ax && !a.flux_in && !a.vmapP)
       return vreg ? launch_valu<NQ, true, true, true>(a, s) : launch_valu<NQ, false, true, true>(a, s);
-    // a given flux (cal_dqdt): the staged kernel, same bits
-    if (vreg && !a.flux_in) return ax ? launch_valu<NQ, true, true>(a, s) : launch_valu<NQ, true, false>(a, s);
+    if (vreg && a.flux_in) {
+      if constexpr (has_gu<NQ, true>())
+        if (!a.geoid) return launch_flux<NQ, true>(a, s);
+      return launch_flux<NQ, false>(a, s);
+    }
+    if (vreg) return ax ? launch_valu<NQ, true, true>(a, s) : launch_valu<NQ, true, false>(a, s);
     return ax ? launch_valu<NQ, false, true>(a, s) : launch_valu<NQ, false, false>(a, s);
   }
   using T = Tile<NQ>;
