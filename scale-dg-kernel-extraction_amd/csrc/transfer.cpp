@@ -28,10 +28,13 @@ constexpr int64_t kWorthPool = (int64_t)48 << 20;
 
 // The pinned chunks, streams and events of one download at a time, shared by
 // every handle of the process (16 MiB): made once kWorthPool bytes have been
-// asked for, given back when the last handle is destroyed.
+// asked for, given back when the last handle is destroyed.  `mu` guards the
+// counts and `busy` and is held for no longer than they take to change; who has
+// set `busy` owns the rest.
 struct Pool {
   std::mutex mu;
   int refs = 0;
+  bool busy = false;   // a download is using or making the chunks
   int device = -1;     // -1: not made
   int64_t plain = 0;   // bytes of large downloads so far, while not made
   char *pinned = nullptr;
@@ -119,47 +122,80 @@ void transfer_retain() {
 
 void transfer_release() {
   std::lock_guard<std::mutex> lk(g_pool.mu);
-  if (--g_pool.refs == 0 && g_pool.device >= 0) free_pool(g_pool);
+  if (--g_pool.refs == 0 && !g_pool.busy && g_pool.device >= 0) free_pool(g_pool);
 }
+
+namespace {
+
+// The pool for one download, if no other has it, it is worth making and it
+// belongs to this device; given back at the end of the scope.
+class Lease {
+ public:
+  Lease(int64_t bytes, int device) {
+    {
+      std::lock_guard<std::mutex> lk(g_pool.mu);
+      if (g_pool.busy || g_pool.refs < 1) return;
+      if (g_pool.device < 0) {
+        g_pool.plain += bytes;
+        if (g_pool.plain < kWorthPool) return;
+      } else if (g_pool.device != device) {
+        return;
+      }
+      g_pool.busy = held_ = true;
+    }
+    usable_ = g_pool.device == device || make_pool(g_pool, device);
+  }
+  ~Lease() {
+    if (!held_) return;
+    std::lock_guard<std::mutex> lk(g_pool.mu);
+    g_pool.busy = false;
+    if (g_pool.refs == 0 && g_pool.device >= 0) free_pool(g_pool);
+  }
+  Lease(const Lease &) = delete;
+  Lease &operator=(const Lease &) = delete;
+  explicit operator bool() const { return usable_; }
+
+ private:
+  bool held_ = false, usable_ = false;
+};
+
+int download_sliced(void *dst, const void *src, int64_t bytes) {
+  int64_t slice = (bytes + kLanes - 1) / kLanes;
+  slice = (slice + 4095) / 4096 * 4096;
+  std::atomic<int> failed{0};
+  auto work = [&](int l) {
+    const int64_t at = l * slice, n = bytes - at < slice ? bytes - at : slice;
+    if (n <= 0) return;
+    const hipError_t e = copy_slice(g_pool, l, (char *)dst + at, (const char *)src + at, n);
+    if (e != hipSuccess) failed.store((int)e);
+  };
+  std::thread t[kLanes];
+  for (int l = 1; l < kLanes; ++l) {
+    try {
+      t[l] = std::thread(work, l);
+    } catch (...) {  // no thread: this one does its slice
+    }
+  }
+  work(0);
+  for (int l = 1; l < kLanes; ++l) {
+    if (t[l].joinable()) t[l].join();
+    else work(l);
+  }
+  if (const int e = failed.load())
+    return set_error(DGK_ERR_DEVICE,
+                     std::string("download: ") + hipGetErrorString((hipError_t)e));
+  return DGK_OK;
+}
+
+}  // namespace
 
 int download(void *dst, const void *src, int64_t bytes, int device, hipStream_t s) {
   if (bytes >= kSliced && pageable(dst)) {
-    std::unique_lock<std::mutex> lk(g_pool.mu, std::try_to_lock);
-    // another download has the pool, it is not made yet, or it belongs to
-    // another device: plain copy
-    bool sliced = lk.owns_lock() && g_pool.refs > 0;
-    if (sliced && g_pool.device < 0) {
-      g_pool.plain += bytes;
-      sliced = g_pool.plain >= kWorthPool && make_pool(g_pool, device);
-    }
-    if (sliced && g_pool.device == device) {
-      DGK_HIP(hipStreamSynchronize(s));
-      int64_t slice = (bytes + kLanes - 1) / kLanes;
-      slice = (slice + 4095) / 4096 * 4096;
-      std::atomic<int> failed{0};
-      auto work = [&](int l) {
-        const int64_t at = l * slice, n = bytes - at < slice ? bytes - at : slice;
-        if (n <= 0) return;
-        const hipError_t e = copy_slice(g_pool, l, (char *)dst + at, (const char *)src + at, n);
-        if (e != hipSuccess) failed.store((int)e);
-      };
-      std::thread t[kLanes];
-      for (int l = 1; l < kLanes; ++l) {
-        try {
-          t[l] = std::thread(work, l);
-        } catch (...) {  // no thread: this one does its slice
-        }
-      }
-      work(0);
-      for (int l = 1; l < kLanes; ++l) {
-        if (t[l].joinable()) t[l].join();
-        else work(l);
-      }
-      if (const int e = failed.load())
-        return set_error(DGK_ERR_DEVICE,
-                         std::string("download: ") + hipGetErrorString((hipError_t)e));
-      return DGK_OK;
-    }
+    // the steps queued before it are waited for with nothing held: other
+    // threads' handles and downloads do not wait for them
+    DGK_HIP(hipStreamSynchronize(s));
+    Lease lease(bytes, device);
+    if (lease) return download_sliced(dst, src, bytes);
   }
   DGK_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s));
   DGK_HIP(hipStreamSynchronize(s));
