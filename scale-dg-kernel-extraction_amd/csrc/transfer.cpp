@@ -122,7 +122,7 @@ void transfer_retain() {
 
 void transfer_release() {
   std::lock_guard<std::mutex> lk(g_pool.mu);
-  if (--g_pool.refs == 0 && !g_pool.busy && g_pool.device >= 0) free_pool(g_pool);
+  if (--g_pool.refs == 0 && !g_pool.busy) free_pool(g_pool);  // and the count starts anew
 }
 
 namespace {
@@ -149,7 +149,7 @@ class Lease {
     if (!held_) return;
     std::lock_guard<std::mutex> lk(g_pool.mu);
     g_pool.busy = false;
-    if (g_pool.refs == 0 && g_pool.device >= 0) free_pool(g_pool);
+    if (g_pool.refs == 0) free_pool(g_pool);
   }
   Lease(const Lease &) = delete;
   Lease &operator=(const Lease &) = delete;

@@ -2,6 +2,7 @@
 // these: device memory is host memory, a copy is a memcpy, and a stream's
 // queued work is a gate that the test opens.  One scenario per run, named on the
 // command line; exit status 0 when it holds.
+#include <algorithm>
 #include <chrono>
 #include <condition_variable>
 #include <cstdio>
@@ -156,11 +157,63 @@ int download_while_waiting() {
   return n == 8 && f.same() ? 0 : fails("a download was copied plainly though no chunk was in use");
 }
 
+// The bytes asked for are counted while a handle lives: a program that makes
+// and destroys its handles starts anew with each.
+int plain_count_ends_with_handles() {
+  Field f(20 * MiB);
+  for (int k = 0; k < 3; ++k) {
+    dgk::transfer_retain();
+    f.get();
+    dgk::transfer_release();
+  }
+  return pinned_allocs == 0 ? 0 : fails("bytes of destroyed handles made the pool");
+}
+
+// Sliced downloads at the sizes where chunks and slices change: every byte, in
+// the number of copies that the slices and chunks make.
+int sliced_sizes() {
+  make_pool();
+  for (int64_t n : {4 * MiB, 4 * MiB + 1, 4 * MiB + 512, 8 * MiB - 1, 8 * MiB, 8 * MiB + 4096,
+                    8 * MiB + 4097, 16 * MiB + 8, 33 * MiB + 77}) {
+    Field f(n);
+    const int before = copies;
+    if (f.get() != 0 || !f.same()) return fails("bytes differ");
+    const int64_t slice = ((n + 7) / 8 + 4095) / 4096 * 4096;
+    int64_t want = 0;
+    for (int64_t at = 0; at < n; at += slice) want += (std::min(slice, n - at) + MiB - 1) / MiB;
+    if (copies - before != want) return fails("not the sliced way");
+  }
+  Field f(4 * MiB - 8);
+  const int before = copies;
+  if (f.get() != 0 || !f.same() || copies - before != 1) return fails("below 4 MiB: one copy");
+  return 0;
+}
+
+// Destinations that are not pageable take one copy; a copy that fails is
+// reported and leaves the pool usable.
+int plain_destinations_and_failures() {
+  make_pool();
+  Field f(8 * MiB);
+  not_pageable.insert(f.dst.data());
+  const int before = copies;
+  if (f.get() != 0 || !f.same() || copies - before != 1) return fails("not one plain copy");
+  not_pageable.clear();
+  fail_copy = copies + 5;
+  if (f.get() == 0) return fails("a failed copy was not reported");
+  fail_copy = -1;
+  if (f.get() != 0 || !f.same()) return fails("no download after a failed one");
+  dgk::transfer_release();
+  return pinned_allocs == 1 && pinned_frees == 1 ? 0 : fails("the pool was not given back");
+}
+
 }  // namespace
 
 int main(int, char **argv) {
   const std::string s = argv[1];
   if (s == "handles_while_waiting") return handles_while_waiting();
   if (s == "download_while_waiting") return download_while_waiting();
+  if (s == "plain_count_ends_with_handles") return plain_count_ends_with_handles();
+  if (s == "sliced_sizes") return sliced_sizes();
+  if (s == "plain_destinations_and_failures") return plain_destinations_and_failures();
   return 2;
 }

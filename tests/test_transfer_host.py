@@ -24,7 +24,9 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["handles_while_waiting", "download_while_waiting"])
+@pytest.mark.parametrize("scenario", ["handles_while_waiting", "download_while_waiting",
+                                      "plain_count_ends_with_handles", "sliced_sizes",
+                                      "plain_destinations_and_failures"])
 def test_scenario(program, scenario):
     r = subprocess.run([str(program), scenario], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
