@@ -519,16 +519,18 @@ int dgk_set_field(dgk_solver *s, int which, const double *f, int64_t n) {
   if (which != DGK_FIELD_Q) {
     DGK_TRY(launch_halo_gather(dst, s->halo, owned, s->NhaloNode, s->stream));
     DGK_TRY(refresh_f32(s, which));
-    // one value everywhere?  The device looks only if a few values agree.
+    // one value everywhere?  The device looks only if a few values agree; it
+    // looks at once at an array that the host cannot read.
     const int d = which - DGK_FIELD_U;
     int32_t varies = 0;
-    for (int64_t k : {owned / 3, owned / 2, owned - 1})
-      varies |= std::memcmp(f + k, f, sizeof(double)) != 0;
+    if (!device_memory(f))
+      for (int64_t k : {owned / 3, owned / 2, owned - 1})
+        varies |= std::memcmp(f + k, f, sizeof(double)) != 0;
     if (!varies) {
       int32_t *flag = (int32_t *)s->mm;
       DGK_TRY(launch_varies(dst, owned, flag, s->stream));
-      DGK_HIP(hipMemcpyAsync(&varies, flag, sizeof(varies), hipMemcpyDeviceToHost, s->stream));
       DGK_TRY(geo_velocity_from_field(s, d));
+      DGK_HIP(hipMemcpyAsync(&varies, flag, sizeof(varies), hipMemcpyDeviceToHost, s->stream));
     }
     DGK_HIP(hipStreamSynchronize(s->stream));
     s->vel_constant[d] = !varies;

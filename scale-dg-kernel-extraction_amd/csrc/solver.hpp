@@ -99,6 +99,8 @@ double *field_ptr(dgk_solver *s, int which);
 // enqueued on `s`, and wait for it (transfer.cpp).  Handles that download hold
 // a reference to the shared staging memory while they live.
 int download(void *dst, const void *src, int64_t bytes, int device, hipStream_t s);
+// Memory that the host's own loads cannot be used on.
+bool device_memory(const void *p);
 void transfer_retain();
 void transfer_release();
 int refresh_f32(dgk_solver *s, int which);

@@ -101,19 +101,23 @@ hipError_t copy_slice(const Pool &p, int l, char *dst, const char *src, int64_t 
   return e;
 }
 
-// Ordinary pageable memory, the only kind the slices are for: the runtime
-// copies straight into pinned memory at the link's rate, and a thread cannot
-// write device memory.
-bool pageable(const void *p) {
+hipMemoryType memory_type(const void *p) {
   hipPointerAttribute_t a;
   if (hipPointerGetAttributes(&a, p) != hipSuccess) {
     (void)hipGetLastError();
-    return true;
+    return hipMemoryTypeUnregistered;
   }
-  return a.type == hipMemoryTypeUnregistered;
+  return a.type;
 }
 
+// Ordinary pageable memory, the only kind the slices are for: the runtime
+// copies straight into pinned memory at the link's rate, and a thread cannot
+// write device memory.
+bool pageable(const void *p) { return memory_type(p) == hipMemoryTypeUnregistered; }
+
 }  // namespace
+
+bool device_memory(const void *p) { return memory_type(p) == hipMemoryTypeDevice; }
 
 void transfer_retain() {
   std::lock_guard<std::mutex> lk(g_pool.mu);
