@@ -54,7 +54,7 @@ struct dgk_solver {
   double *geo = nullptr, *D = nullptr, *Lift = nullptr;
   uint32_t *geoid = nullptr;
   double *mm = nullptr;       // min/max partials, then the block counter
-  double *mm_host = nullptr;  // pinned: min, max (made by the first dgk_minmax)
+  double *mm_host = nullptr;  // pinned: min, max (handles that have dgk_minmax)
   bool set[4] = {false, false, false, false};
   int64_t bytes = 0;
   std::vector<void *> allocs;
