@@ -300,8 +300,9 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * that has not been autotuned; dgk_tile_selected reports the choice for
  * launches with velocity fields.  Launches with a given flux (dgk_cal_dqdt)
  * or a stored, non-separable Lift always use the VALU kernels.  dgk_autotune
- * times each candidate with HIP events over reps RK-stage launches on the
- * solver's own mesh (writing only the solver's scratch rotation buffer) and
+ * times each candidate with HIP events over the stage launches of whole steps,
+ * at least reps of them, on the solver's own mesh (writing only its scratch
+ * rotation buffers) and
  * keeps the fastest for that solver alone, since the best shape depends on
  * the mesh (the solver's default stays unless another shape is at least 2%
  * faster);

@@ -1193,9 +1193,10 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls) {
 // Tile shapes and the autotuner.  A stage kernel has one or more tile shapes
 // per order (elements per workgroup); the selection is per process, per form
 // and order.  The autotuner times every candidate on a solver's own mesh with
-// HIP events around `reps` RK-stage launches (stage-2 configuration: RK base
-// read, output to the solver's scratch rotation buffer) and keeps the
-// fastest.  Per-element arithmetic does not depend on the shape.
+// HIP events around the stage launches of whole steps, at least `reps` of them,
+// and keeps the fastest.  The last stage writes the scratch rotation buffer that
+// the first one did, so the field stays.  Per-element arithmetic does not depend on
+// the shape.
 // ---------------------------------------------------------------------------
 namespace {
 
@@ -1230,22 +1231,33 @@ int solver_selected(const dgk_solver *s) {
                                         : stage_f64_selected_cvel(s->Nq);
 }
 
+// One step's stage launches of s into its scratch rotation buffers: the inputs, RK
+// bases and outputs of dgk_step, but for the last output.
+int scratch_step(dgk_solver *s) {
+  double *A = s->q[s->cur], *B = s->q[(s->cur + 1) % 3], *C = s->q[(s->cur + 2) % 3];
+  const double *in[3] = {A, B, C};
+  double *out[3] = {B, C, B};
+  for (int st = 0; st < 3; ++st)
+    DGK_TRY(launch_stage(s, in[st], A, out[st], 1, kRkA[st], kRkB[st], 0.0));
+  return DGK_OK;
+}
+
 // Average device time of one stage launch of s, in microseconds.
 int time_stage(dgk_solver *s, int reps, double *us) {
-  double *A = s->q[s->cur], *C = s->q[(s->cur + 2) % 3];
   hipEvent_t a = nullptr, b = nullptr;
   DGK_HIP(hipEventCreate(&a));
   DGK_HIP(hipEventCreate(&b));
-  int rc = launch_stage(s, A, A, C, 1, kRkA[1], kRkB[1], 0.0);
+  const int steps = reps / 3 + (reps % 3 != 0);
+  int rc = scratch_step(s);
   if (rc == DGK_OK && hipEventRecord(a, s->stream) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event");
-  for (int r = 0; r < reps && rc == DGK_OK; ++r) rc = launch_stage(s, A, A, C, 1, kRkA[1], kRkB[1], 0.0);
+  for (int r = 0; r < steps && rc == DGK_OK; ++r) rc = scratch_step(s);
   if (rc == DGK_OK && hipEventRecord(b, s->stream) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event");
   if (rc == DGK_OK && hipEventSynchronize(b) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event sync");
   float ms = 0.f;
   if (rc == DGK_OK && hipEventElapsedTime(&ms, a, b) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "elapsed");
   (void)hipEventDestroy(a);
   (void)hipEventDestroy(b);
-  if (rc == DGK_OK) *us = 1e3 * ms / reps;
+  if (rc == DGK_OK) *us = 1e3 * ms / (3.0 * steps);
   return rc;
 }
 
@@ -1253,7 +1265,7 @@ constexpr double kTuneMargin = 0.02;
 
 // Whether candidate c launches its own kernel for s's stage launches.
 bool candidate_runs(dgk_solver *s, int c) {
-  double *A = s->q[s->cur], *C = s->q[(s->cur + 2) % 3];
+  double *A = s->q[s->cur], *C = s->q[(s->cur + 2) % 3];  // the three are aligned alike
   if (s->evaltype == DGK_EVAL_HIP_MP) {
     StageArgsMP a = stage_args_mp(s, A, A, C, 1, kRkA[1], kRkB[1], 0.0);
     return stage_mp_candidate_runs(s->Nq, c, a);
