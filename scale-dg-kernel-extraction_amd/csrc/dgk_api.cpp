@@ -1232,25 +1232,27 @@ int solver_selected(const dgk_solver *s) {
 }
 
 // One step's stage launches of s into its scratch rotation buffers: the inputs, RK
-// bases and outputs of dgk_step, but for the last output.
-int scratch_step(dgk_solver *s) {
+// bases and outputs of dgk_step, but for the last output.  dt_geo as the launches
+// that are to be timed (a batch's take the time step from the geometry records, and
+// with it the kernels' way to a record that the workgroup shares).
+int scratch_step(dgk_solver *s, int dt_geo) {
   double *A = s->q[s->cur], *B = s->q[(s->cur + 1) % 3], *C = s->q[(s->cur + 2) % 3];
   const double *in[3] = {A, B, C};
   double *out[3] = {B, C, B};
   for (int st = 0; st < 3; ++st)
-    DGK_TRY(launch_stage(s, in[st], A, out[st], 1, kRkA[st], kRkB[st], 0.0));
+    DGK_TRY(launch_stage(s, in[st], A, out[st], 1, kRkA[st], kRkB[st], 0.0, nullptr, dt_geo));
   return DGK_OK;
 }
 
 // Average device time of one stage launch of s, in microseconds.
-int time_stage(dgk_solver *s, int reps, double *us) {
+int time_stage(dgk_solver *s, int reps, int dt_geo, double *us) {
   hipEvent_t a = nullptr, b = nullptr;
   DGK_HIP(hipEventCreate(&a));
   DGK_HIP(hipEventCreate(&b));
   const int steps = reps / 3 + (reps % 3 != 0);
-  int rc = scratch_step(s);
+  int rc = scratch_step(s, dt_geo);
   if (rc == DGK_OK && hipEventRecord(a, s->stream) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event");
-  for (int r = 0; r < steps && rc == DGK_OK; ++r) rc = scratch_step(s);
+  for (int r = 0; r < steps && rc == DGK_OK; ++r) rc = scratch_step(s, dt_geo);
   if (rc == DGK_OK && hipEventRecord(b, s->stream) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event");
   if (rc == DGK_OK && hipEventSynchronize(b) != hipSuccess) rc = set_error(DGK_ERR_DEVICE, "event sync");
   float ms = 0.f;
@@ -1273,7 +1275,7 @@ bool candidate_runs(dgk_solver *s, int c) {
   return stage_f64_candidate_runs(s->Nq, c, stage_args(s, A, A, C, 1, kRkA[1], kRkB[1], 0.0));
 }
 
-int autotune(dgk_solver *s, int reps, int *best, double *us, int max, int *n) {
+int autotune(dgk_solver *s, int reps, int dt_geo, int *best, double *us, int max, int *n) {
   int epb[kMaxTileShapes];
   const int nc = tile_shapes(s->evaltype, s->Nq, epb);
   if (nc < 1) return set_error(DGK_ERR_UNSUPPORTED, "no tile shapes for this form and order");
@@ -1286,7 +1288,7 @@ int autotune(dgk_solver *s, int reps, int *best, double *us, int max, int *n) {
       continue;
     }
     s->tile = c;
-    const int rc = time_stage(s, reps, &t[c]);
+    const int rc = time_stage(s, reps, dt_geo, &t[c]);
     if (rc != DGK_OK) {
       s->tile = -1;
       return rc;
@@ -1345,7 +1347,7 @@ int dgk_autotune(dgk_solver *s, int reps, int *best, double *us_per_launch, int 
   DGK_TRY(enter(s));
   DGK_TRY(require_fields(s));
   if (reps < 1) return set_error(DGK_ERR_ARG, "reps must be >= 1");
-  return autotune(s, reps, best, us_per_launch, max, n);
+  return autotune(s, reps, 0, best, us_per_launch, max, n);
 }
 
 int dgk_batch_autotune(dgk_batch *b, int reps, int *p, int *best, double *us_best,
@@ -1360,7 +1362,7 @@ int dgk_batch_autotune(dgk_batch *b, int reps, int *p, int *best, double *us_bes
     dgk_solver *s = b->groups[g];
     double t[kMaxTileShapes] = {};
     int arg = 0, nc = 0;
-    DGK_TRY(autotune(s, reps, &arg, t, kMaxTileShapes, &nc));
+    DGK_TRY(autotune(s, reps, 1, &arg, t, kMaxTileShapes, &nc));
     if ((int)g < max) {
       if (p) p[g] = b->group_p[g];
       if (best) best[g] = arg;

@@ -33,3 +33,27 @@ def test_solver_times_are_the_steps(form, p, ne):
             seconds, n = s.timers()["Stage (fused)"]
             steps.append(1e6 * seconds / n)
     assert abs(tuned - min(steps)) < WITHIN * min(steps), (steps, runs)
+
+
+@pytest.mark.parametrize("form,p,ne", [("HIP_MP", 2, 85), ("HIP", 3, 64), ("HIP", 7, 32)])
+def test_batch_times_are_the_steps(form, p, ne):
+    """A batch's launches read a workgroup's geometry record as scalars; timed as
+    a solver's launches they took the per-lane reads (mixed p = 2, 125 against
+    106 us in the step)."""
+    with dgk.Batch(form, [dict(ne=(ne, ne, ne), p=p, dt=1e-5)]) as b:
+        b.init_gaussian(0, (0.3, 0.4, 0.5), 0.1, VEL)
+        b.step(20)
+        b.synchronize()
+        before = b.get_field(0)
+        runs = [b.autotune(reps=60) for _ in range(3)]
+        assert (b.get_field(0) == before).all()
+        tuned = min(r[0]["us_per_launch"] for r in runs if r[0]["candidate"] == runs[-1][0]["candidate"])
+        b.step(20)
+        steps = []
+        for _ in range(3):
+            b.synchronize()
+            b.timer()
+            b.step(40)
+            seconds, _ = b.timer()
+            steps.append(1e6 * seconds / 120)
+    assert abs(tuned - min(steps)) < WITHIN * min(steps), (steps, runs)
