@@ -558,9 +558,11 @@ stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restr
   auto body = [&](const double *__restrict__ g) {
     double cvel[3] = {0.0, 0.0, 0.0};
     if constexpr (CVEL) {
-      cvel[0] = g[kGeoVel];
-      cvel[1] = g[kGeoVel + 1];
-      cvel[2] = g[kGeoVel + 2];
+      // as the fields hold it: FP32 in the mixed form (a batch's and a request's
+      // record has the FP64 value)
+      cvel[0] = (double)(VT)g[kGeoVel];
+      cvel[1] = (double)(VT)g[kGeoVel + 1];
+      cvel[2] = (double)(VT)g[kGeoVel + 2];
     }
     // flux of this lane's node of face f
     auto face_flux = [&](int f, double qM, double vm) {
