@@ -293,8 +293,9 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * add the same products in the same order on the VALU (the same bits, faster),
  * and all at once and direction by direction then are one kernel; the MFMA
  * itself runs direction-by-direction launches of the mixed form at p = 16, 17,
- * and constant-velocity ones of the mixed form at p >= 16 and of FP64 at
- * p = 16.
+ * constant-velocity ones of the mixed form at p >= 16 and of FP64 at p = 16, and
+ * the mixed form's launches of at most 256 elements (512 with a constant
+ * velocity) at p = 13..15, all at once, whatever the candidate.
  * dgk_tile_select sets the process-wide choice for that form and order, for
  * both kinds of launch (-1 restores the defaults); it holds for every solver
  * that has not been autotuned; dgk_tile_selected reports the choice for

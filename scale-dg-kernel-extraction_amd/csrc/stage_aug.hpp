@@ -39,7 +39,8 @@
 //    faster (by_mfma): mixed p = 16, 17 (fields 140 against 177 and 137 against
 //    158) and constant-velocity launches of the mixed form at p >= 16 (101
 //    against 139, 104/127, 100/113, 110/130) and of FP64 at p = 16 (133/150).
-//    There an element is five to seven wavefronts, and on four SIMDs the VALU
+//    and launches of few elements of the mixed form at p = 13..15 (stage_small).
+//    Above p = 15 an element is five to seven wavefronts, and on four SIMDs the VALU
 //    form's phases take as long as two of them, while the MFMA form's eight
 //    wavefronts share the tiles.
 #pragma once
@@ -121,7 +122,9 @@ struct Seq {
   // (rows of 4 KSTEPS: 79% of the LDS cycles were conflicts at p = 18).  The K
   // padding is not stored: the operand read puts zeros there.
   static constexpr int STRIDE = KAUG | 1;
-  static constexpr size_t LDS_BYTES = (size_t)(ROWS * STRIDE + 4) * sizeof(typename P::op_t);
+  static constexpr int AREA = ROWS * STRIDE;               // A of one direction
+  static constexpr size_t LDS_BYTES = (size_t)(AREA + 4) * sizeof(typename P::op_t);
+  static constexpr size_t LDS_BYTES_ONCE = (size_t)(3 * AREA + 4) * sizeof(typename P::op_t);
   static constexpr int JPW = (MTILES + WAVES - 1) / WAVES;
 };
 
@@ -508,157 +511,182 @@ stage_aug(const double *__restrict__ q_, const double *q0_,
 //      rows l = kq*KSTEPS + ks of B in registers and reads A at fixed offsets
 //      from its own base; the result overwrites the tile's rows in place;
 //   4. the direction results are summed in FP64 and RK-combined.
-// AXAL: every face normal lies along its face's axis (checked on the host);
-// the ax_runtime shapes test it at run time (instantiated as the general form).
-// CVEL: constant velocity per element, (u, v, w) = words kGeoVel..+2 of its
-// geometry record (batched and served boxes, solvers with constant fields); no
-// velocity field is read, and the operand-precision value of a constant is the
-// value its per-node copy holds, so the results are the same bits.
-// GU: several elements per workgroup and one geometry record for the whole
-// launch (no per-element record ids): the record is read through the kernel
-// argument itself, i.e. through the scalar cache (as in stage_f64).
-template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL = false, bool GU = false>
-__global__ void
-__attribute__((amdgpu_flat_work_group_size(1, Shape<P, NQ, EPB, SEQ, CVEL>::THREADS),
-               amdgpu_waves_per_eu(Shape<P, NQ, EPB, SEQ, CVEL>::MIN_WAVES_EU)))
-stage_mfma(const double *__restrict__ q_, const double *q0_,
-           const typename P::vel_t *__restrict__ u_, const typename P::vel_t *__restrict__ v_,
-           const typename P::vel_t *__restrict__ w_, double *out_,
-           const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
-           const typename P::op_t *__restrict__ D_, const typename P::op_t *__restrict__ ell_,
-           const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
-           const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
-           const double cb_, const double dt_, const int mode_, const int axis_aligned_,
-           const int dt_geo_, const int rev_, const int64_t zp_) {
-  static_assert(!GU || EPB > 1, "one element per workgroup reads its record uniformly anyway");
-  if constexpr (!Shape<P, NQ, EPB, SEQ, CVEL>::MFMA) {
-    stage_aug<P, NQ, EPB, ax_runtime<P, NQ, EPB, SEQ>(), AXAL, CVEL, GU>(
-        q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_, geoid_, order_, Ne_, ca_, cb_,
-        dt_, mode_, axis_aligned_, dt_geo_, rev_, zp_);
-  } else {
-    using C = Seq<P, NQ>;
-    using vel_t = typename P::vel_t;
-    using op_t = typename P::op_t;
-    constexpr int NQ2 = C::NQ2, NP = C::NP, NFT = 6 * NQ2, KSTEPS = C::KSTEPS;
-    constexpr int KAUG = C::KAUG, STRIDE = C::STRIDE;
-    extern __shared__ double smem_mp[];
-    op_t *const As = (op_t *)smem_mp;
+// ONCE: the three directions at once, each in an LDS area of its own, their velocity
+// columns loaded with the rest.
+template <class P, int NQ, bool CVEL, bool ONCE>
+__device__ __forceinline__ void
+stage_seq(const double *q_, const double *q0_,
+          const typename P::vel_t *u_, const typename P::vel_t *v_,
+          const typename P::vel_t *w_, double *out_,
+          const int32_t *nbr_, const int32_t *vmapP_,
+          const typename P::op_t *D_, const typename P::op_t *ell_,
+          const double *geo_, const uint32_t *geoid_,
+          const int32_t *order_, const int64_t Ne_, const double ca_,
+          const double cb_, const double dt_, const int mode_, const int axis_aligned_,
+          const int dt_geo_, const int rev_, const int64_t zp_) {
+  using C = Seq<P, NQ>;
+  using vel_t = typename P::vel_t;
+  using op_t = typename P::op_t;
+  constexpr int NQ2 = C::NQ2, NP = C::NP, NFT = 6 * NQ2, KSTEPS = C::KSTEPS;
+  constexpr int KAUG = C::KAUG, STRIDE = C::STRIDE;
+  extern __shared__ double smem_mp[];
+  op_t *const As = (op_t *)smem_mp;
 
-    const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int64_t slot = (int64_t)xcd_block_mp(blockIdx.x, gridDim.x);
-    const bool lane_ok = tid < NQ2;
-    const int ij = lane_ok ? tid : 0;
-    const int i = ij % NQ, j = ij / NQ;
-    const bool active = lane_ok && slot < Ne_;
-    int64_t e = slot < Ne_ ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
-    e = uniform_mp(e);
-    const double *__restrict__ g = geo_ + (geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
-    const int64_t ebase = e * NP;
-    const int64_t base = ebase + ij;
-    const bool rk = mode_ == 1;
-    const bool use_q0 = rk && ca_ != 0.0;
-    const bool axal = axis_aligned_ != 0;
-    const vel_t *const velp[3] = {u_, v_, w_};
-    vel_t cv[3] = {(vel_t)0, (vel_t)0, (vel_t)0};
-    if constexpr (CVEL) {
-      cv[0] = (vel_t)g[kGeoVel];
-      cv[1] = (vel_t)g[kGeoVel + 1];
-      cv[2] = (vel_t)g[kGeoVel + 2];
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6, lane = tid & 63;
+  const int64_t slot = (int64_t)xcd_block_mp(blockIdx.x, gridDim.x);
+  const bool lane_ok = tid < NQ2;
+  const int ij = lane_ok ? tid : 0;
+  const int i = ij % NQ, j = ij / NQ;
+  const bool active = lane_ok && slot < Ne_;
+  int64_t e = slot < Ne_ ? slot_element(slot, Ne_, order_, rev_, zp_) : 0;
+  e = uniform_mp(e);
+  const double *__restrict__ g = geo_ + (geoid_ ? (int64_t)geoid_[e] * kGeoStride : 0);
+  const int64_t ebase = e * NP;
+  const int64_t base = ebase + ij;
+  const bool rk = mode_ == 1;
+  const bool use_q0 = rk && ca_ != 0.0;
+  const bool axal = axis_aligned_ != 0;
+  const vel_t *const velp[3] = {u_, v_, w_};
+  vel_t cv[3] = {(vel_t)0, (vel_t)0, (vel_t)0};
+  if constexpr (CVEL) {
+    cv[0] = (vel_t)g[kGeoVel];
+    cv[1] = (vel_t)g[kGeoVel + 1];
+    cv[2] = (vel_t)g[kGeoVel + 2];
+  }
+  auto nbr_at = [&](int f) -> int64_t {
+    return vmapP_ ? (int64_t)vmapP_[e * NFT + f * NQ2 + ij]
+                  : (int64_t)nbr_[e * 6 + f] * NP + nbr_face_node(f, i, j, NQ);
+  };
+
+  // ---- 1. loads straight into registers ------------------------------------
+  double qc[NQ], qM[4], qP[6];
+  vel_t w0 = cv[2], w1 = cv[2], vM[4], vP[6];  // velocity component along the face axis
+  vel_t cols[3][NQ];                           // ONCE: the velocity columns
+  if (active) {
+#pragma unroll
+    for (int k = 0; k < NQ; ++k) qc[k] = q_[base + k * NQ2];
+    if constexpr (ONCE && !CVEL) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) cols[d][k] = velp[d][base + k * NQ2];
     }
-    auto nbr_at = [&](int f) -> int64_t {
-      return vmapP_ ? (int64_t)vmapP_[e * NFT + f * NQ2 + ij]
-                    : (int64_t)nbr_[e * 6 + f] * NP + nbr_face_node(f, i, j, NQ);
-    };
-
-    // ---- 1. loads straight into registers ------------------------------------
-    double qc[NQ], qM[4], qP[6];
-    vel_t w0 = cv[2], w1 = cv[2], vM[4], vP[6];  // velocity component along the face axis
-    if (active) {
-#pragma unroll
-      for (int k = 0; k < NQ; ++k) qc[k] = q_[base + k * NQ2];
-      if constexpr (!CVEL) {
-        w0 = w_[base];
-        w1 = w_[base + (NQ - 1) * NQ2];
-      }
-#pragma unroll
-      for (int f = 0; f < 4; ++f) {  // own traces of the x and y faces
-        const int64_t m = ebase + own_face_node(f, i, j, NQ);
-        qM[f] = q_[m];
-        vM[f] = CVEL ? cv[kFaceAxis[f]] : (kFaceAxis[f] == 0 ? u_ : v_)[m];
-      }
-#pragma unroll
-      for (int f = 0; f < 6; ++f) {
-        const int64_t pidx = nbr_at(f);
-        qP[f] = q_[pidx];
-        vP[f] = CVEL ? cv[kFaceAxis[f]]
-                     : (kFaceAxis[f] == 0 ? u_ : kFaceAxis[f] == 1 ? v_ : w_)[pidx];
-      }
+    if constexpr (!CVEL) {
+      w0 = w_[base];
+      w1 = w_[base + (NQ - 1) * NQ2];
     }
+#pragma unroll
+    for (int f = 0; f < 4; ++f) {  // own traces of the x and y faces
+      const int64_t m = ebase + own_face_node(f, i, j, NQ);
+      qM[f] = q_[m];
+      vM[f] = CVEL ? cv[kFaceAxis[f]] : (kFaceAxis[f] == 0 ? u_ : v_)[m];
+    }
+#pragma unroll
+    for (int f = 0; f < 6; ++f) {
+      const int64_t pidx = nbr_at(f);
+      qP[f] = q_[pidx];
+      vP[f] = CVEL ? cv[kFaceAxis[f]]
+                   : (kFaceAxis[f] == 0 ? u_ : kFaceAxis[f] == 1 ? v_ : w_)[pidx];
+    }
+  }
 
-    // ---- 2a. FP64 upwind fluxes -------------------------------------------------
-    op_t fl[6];
-    auto face_flux = [&](int f) {
-      const double qm = f == 4 ? qc[0] : f == 5 ? qc[NQ - 1] : qM[f];
-      double VelM, VelP;
-      if (axal) {
-        const int ax = kFaceAxis[f];
-        const double na = g[kGeoNormal + 3 * f + ax];
-        const vel_t vm = f == 4 ? w0 : f == 5 ? w1 : vM[f];
-        VelM = (double)vm * na;
-        VelP = (double)vP[f] * na;
+  // ---- 2a. FP64 upwind fluxes -------------------------------------------------
+  op_t fl[6];
+  auto face_flux = [&](int f) {
+    const double qm = f == 4 ? qc[0] : f == 5 ? qc[NQ - 1] : qM[f];
+    double VelM, VelP;
+    if (axal) {
+      const int ax = kFaceAxis[f];
+      const double na = g[kGeoNormal + 3 * f + ax];
+      const vel_t vm = f == 4 ? w0 : f == 5 ? w1 : vM[f];
+      VelM = (double)vm * na;
+      VelP = (double)vP[f] * na;
+    } else {
+      // general normals: all three components on both sides
+      const int64_t m = ebase + own_face_node(f, i, j, NQ);
+      const int64_t pidx = nbr_at(f);
+      const double n1 = g[kGeoNormal + 3 * f], n2 = g[kGeoNormal + 3 * f + 1],
+                   n3 = g[kGeoNormal + 3 * f + 2];
+      if constexpr (CVEL) {
+        VelM = (double)cv[0] * n1 + (double)cv[1] * n2 + (double)cv[2] * n3;
+        VelP = VelM;
+        (void)m;
+        (void)pidx;
       } else {
-        // general normals: all three components on both sides
-        const int64_t m = ebase + own_face_node(f, i, j, NQ);
-        const int64_t pidx = nbr_at(f);
-        const double n1 = g[kGeoNormal + 3 * f], n2 = g[kGeoNormal + 3 * f + 1],
-                     n3 = g[kGeoNormal + 3 * f + 2];
-        if constexpr (CVEL) {
-          VelM = (double)cv[0] * n1 + (double)cv[1] * n2 + (double)cv[2] * n3;
-          VelP = VelM;
-          (void)m;
-          (void)pidx;
-        } else {
-          VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
-          VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
-        }
+        VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
+        VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
       }
-      const double alpha = 0.5 * fabs(VelP + VelM);
-      fl[f] = (op_t)(0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qm * VelM - alpha * (qP[f] - qm)));
-    };
+    }
+    const double alpha = 0.5 * fabs(VelP + VelM);
+    fl[f] = (op_t)(0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qm * VelM - alpha * (qP[f] - qm)));
+  };
+  if (active) {
+#pragma unroll
+    for (int f = 0; f < 6; ++f) face_flux(f);
+  }
+
+  // B = [D^T ; l- ; l+ ; 0] rows of this lane (k permuted, see above)
+  constexpr int NT = C::NT;
+  const int col = lane & 15, kq = lane >> 4;
+  op_t bop[NT][KSTEPS];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    const int c = 16 * nt + col;
+#pragma unroll
+    for (int ks = 0; ks < KSTEPS; ++ks) {
+      const int l = kq * KSTEPS + ks;
+      bop[nt][ks] = c >= NQ ? (op_t)0 : l < NQ ? D_[c + l * NQ] : l == NQ ? ell_[c]
+                    : l == NQ + 1 ? ell_[NQ + c] : (op_t)0;
+    }
+  }
+  const int rd = col * STRIDE + kq * KSTEPS;        // A read offset of this lane in a tile
+  const int wr = P::RSTRIDE_Q * kq * STRIDE + col;  // result offset of value 0
+  const int left = KAUG - kq * KSTEPS;              // stored operands of the lane's K range
+  // Node (i,j,k) sits in the x pencil (j,k) at position i, in the y pencil
+  // (i,k) at position j and in the z pencil (i,j) at position k; face node
+  // (i,j) of the faces normal to d is pencil ij of direction d.
+  const int pos_off[3] = {j * STRIDE + i, i * STRIDE + j, ij * STRIDE};
+  const int pos_step[3] = {NQ * STRIDE, NQ * STRIDE, 1};
+  const int face_m[3] = {3, 0, 4}, face_p[3] = {1, 2, 5};  // -d and +d faces
+
+  // ---- 2b-4a, one direction at a time through one LDS area -------------------
+  // Rows of A beyond the element's pencils hold stale LDS; each output row
+  // depends only on its own A row, and those rows are never read back.
+  double tend[NQ], q0v[NQ];
+  if constexpr (ONCE) {
     if (active) {
 #pragma unroll
-      for (int f = 0; f < 6; ++f) face_flux(f);
-    }
-
-    // B = [D^T ; l- ; l+ ; 0] rows of this lane (k permuted, see above)
-    constexpr int NT = C::NT;
-    const int col = lane & 15, kq = lane >> 4;
-    op_t bop[NT][KSTEPS];
+      for (int d = 0; d < 3; ++d) {
+        const double Ed = g[kGeoEscale + d];
+        op_t *a = As + d * C::AREA + pos_off[d];
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int c = 16 * nt + col;
+        for (int k = 0; k < NQ; ++k)
+          a[k * pos_step[d]] = (op_t)(Ed * (qc[k] * (double)(CVEL ? cv[d] : cols[d][k])));
+        op_t *r = As + d * C::AREA + ij * STRIDE;
+        r[NQ] = fl[face_m[d]];
+        r[NQ + 1] = fl[face_p[d]];
+      }
+      if (use_q0) {
 #pragma unroll
-      for (int ks = 0; ks < KSTEPS; ++ks) {
-        const int l = kq * KSTEPS + ks;
-        bop[nt][ks] = c >= NQ ? (op_t)0 : l < NQ ? D_[c + l * NQ] : l == NQ ? ell_[c]
-                      : l == NQ + 1 ? ell_[NQ + c] : (op_t)0;
+        for (int k = 0; k < NQ; ++k) q0v[k] = __builtin_nontemporal_load(q0_ + base + k * NQ2);
       }
     }
-    const int rd = col * STRIDE + kq * KSTEPS;        // A read offset of this lane in a tile
-    const int wr = P::RSTRIDE_Q * kq * STRIDE + col;  // result offset of value 0
-    const int left = KAUG - kq * KSTEPS;              // stored operands of the lane's K range
-    // Node (i,j,k) sits in the x pencil (j,k) at position i, in the y pencil
-    // (i,k) at position j and in the z pencil (i,j) at position k; face node
-    // (i,j) of the faces normal to d is pencil ij of direction d.
-    const int pos_off[3] = {j * STRIDE + i, i * STRIDE + j, ij * STRIDE};
-    const int pos_step[3] = {NQ * STRIDE, NQ * STRIDE, 1};
-    const int face_m[3] = {3, 0, 4}, face_p[3] = {1, 2, 5};  // -d and +d faces
-
-    // ---- 2b-4a, one direction at a time through one LDS area -------------------
-    // Rows of A beyond the element's pencils hold stale LDS; each output row
-    // depends only on its own A row, and those rows are never read back.
-    double tend[NQ];
+    __syncthreads();
+#pragma unroll
+    for (int t = wave; t < 3 * C::MTILES; t += C::WAVES)  // wave-uniform
+      mfma_tile<P, KSTEPS, KAUG, STRIDE, NQ, NT>(As + t * 16 * STRIDE, bop, rd, wr, col, left);
+    __syncthreads();
+    if (active) {
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+          const double x = (double)As[d * C::AREA + pos_off[d] + k * pos_step[d]];
+          tend[k] = d == 0 ? x : tend[k] + x;
+        }
+    }
+  } else {
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
       if (active) {
@@ -696,30 +724,82 @@ stage_mfma(const double *__restrict__ q_, const double *q0_,
       }
       if (d < 2) __syncthreads();  // the next direction overwrites the area
     }
+  }
 
-    // ---- 4b. RK epilogue (FP64).  The RK base is read only here: held through
-    // the last direction's product it cost p = 16, 17 a wave per SIMD.  In a
-    // block of its own, or the allocation spills.
-    double q0v[NQ];
-    if (active && use_q0) {
+  // ---- 4b. RK epilogue (FP64).  The RK base is read only here: held through
+  // the last direction's product it cost p = 16, 17 a wave per SIMD.  In a
+  // block of its own, or the allocation spills.
+  if (!ONCE && active && use_q0) {
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) q0v[k] = __builtin_nontemporal_load(q0_ + base + k * NQ2);
-    }
-    if (active) {
-      const double dtv = dt_geo_ ? g[kGeoDt] : dt_;
+    for (int k = 0; k < NQ; ++k) q0v[k] = __builtin_nontemporal_load(q0_ + base + k * NQ2);
+  }
+  if (active) {
+    const double dtv = dt_geo_ ? g[kGeoDt] : dt_;
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        const double td = -tend[k];
-        const int64_t idx = base + (int64_t)k * NQ2;
-        double res = td;
-        if (rk) {
-          const double upd = cb_ * (qc[k] + dtv * td);
-          res = use_q0 ? ca_ * q0v[k] + upd : upd;
-        }
-        __builtin_nontemporal_store(res, out_ + idx);
+    for (int k = 0; k < NQ; ++k) {
+      const double td = -tend[k];
+      const int64_t idx = base + (int64_t)k * NQ2;
+      double res = td;
+      if (rk) {
+        const double upd = cb_ * (qc[k] + dtv * td);
+        res = use_q0 ? ca_ * q0v[k] + upd : upd;
       }
+      __builtin_nontemporal_store(res, out_ + idx);
     }
   }
+}
+
+// AXAL: every face normal lies along its face's axis (checked on the host);
+// the ax_runtime shapes test it at run time (instantiated as the general form).
+// CVEL: constant velocity per element, (u, v, w) = words kGeoVel..+2 of its
+// geometry record (batched and served boxes, solvers with constant fields); no
+// velocity field is read, and the operand-precision value of a constant is the
+// value its per-node copy holds, so the results are the same bits.
+// GU: several elements per workgroup and one geometry record for the whole
+// launch (no per-element record ids): the record is read through the kernel
+// argument itself, i.e. through the scalar cache (as in stage_f64).
+template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL = false, bool GU = false>
+__global__ void
+__attribute__((amdgpu_flat_work_group_size(1, Shape<P, NQ, EPB, SEQ, CVEL>::THREADS),
+               amdgpu_waves_per_eu(Shape<P, NQ, EPB, SEQ, CVEL>::MIN_WAVES_EU)))
+stage_mfma(const double *__restrict__ q_, const double *q0_,
+           const typename P::vel_t *__restrict__ u_, const typename P::vel_t *__restrict__ v_,
+           const typename P::vel_t *__restrict__ w_, double *out_,
+           const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
+           const typename P::op_t *__restrict__ D_, const typename P::op_t *__restrict__ ell_,
+           const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
+           const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
+           const double cb_, const double dt_, const int mode_, const int axis_aligned_,
+           const int dt_geo_, const int rev_, const int64_t zp_) {
+  static_assert(!GU || EPB > 1, "one element per workgroup reads its record uniformly anyway");
+  if constexpr (!Shape<P, NQ, EPB, SEQ, CVEL>::MFMA) {
+    stage_aug<P, NQ, EPB, ax_runtime<P, NQ, EPB, SEQ>(), AXAL, CVEL, GU>(
+        q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_, geoid_, order_, Ne_, ca_, cb_,
+        dt_, mode_, axis_aligned_, dt_geo_, rev_, zp_);
+  } else {
+    stage_seq<P, NQ, CVEL, false>(
+        q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_, geoid_, order_, Ne_, ca_, cb_,
+        dt_, mode_, axis_aligned_, dt_geo_, rev_, zp_);
+  }
+}
+
+// Launches of few elements (has_small): the MFMA form, the directions at once.
+template <class P, int NQ, bool CVEL>
+__global__ void
+__attribute__((amdgpu_flat_work_group_size(1, Seq<P, NQ>::THREADS),
+               amdgpu_waves_per_eu(CVEL ? 4 : 2)))
+stage_small(const double *__restrict__ q_, const double *q0_,
+            const typename P::vel_t *__restrict__ u_, const typename P::vel_t *__restrict__ v_,
+            const typename P::vel_t *__restrict__ w_, double *out_,
+            const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
+            const typename P::op_t *__restrict__ D_, const typename P::op_t *__restrict__ ell_,
+            const double *__restrict__ geo_, const uint32_t *__restrict__ geoid_,
+            const int32_t *__restrict__ order_, const int64_t Ne_, const double ca_,
+            const double cb_, const double dt_, const int mode_, const int axis_aligned_,
+            const int dt_geo_, const int rev_, const int64_t zp_) {
+  stage_seq<P, NQ, CVEL, true>(q_, q0_, u_, v_, w_, out_, nbr_, vmapP_, D_, ell_, geo_, geoid_,
+                               order_, Ne_, ca_, cb_, dt_, mode_, axis_aligned_, dt_geo_, rev_,
+                               zp_);
 }
 
 template <class P, int NQ, int EPB, bool SEQ, bool AXAL, bool CVEL, bool GU>
@@ -778,11 +858,42 @@ int launch_form(const Args &a, hipStream_t s) {
   return launch_kernel<P, NQ, EPB, SEQ, AXAL, CVEL, false>(a, s);
 }
 
+// Where a launch of few elements takes stage_small: the mixed form at p = 13..15 with
+// at most one element per CU, with a constant velocity two.  Such a launch lasts as
+// long as one element does, which is four wavefronts in the VALU form and eight here,
+// with the three directions between two barriers.  us per launch, stage_aug against
+// stage_small: p = 13 8 elements 7.8/7.2, 256 8.7/8.2, constant velocity 256
+// 8.7/6.7, 512 11.4/10.5; p = 15 8 elements 8.8/8.2, 256 10.2/9.9, constant
+// velocity 256 9.3/7.8, 512 13.8/13.0.  With more elements than that fit at once
+// stage_aug has the higher rate: p = 15 320 elements 14.0/17.5, constant velocity
+// 768 16.9/19.6.  The same bits.
+constexpr int64_t kCus = 256;
+template <class P, int NQ, int EPB>
+constexpr bool has_small() {
+  return sizeof(typename P::op_t) == 4 && NQ >= 14 && NQ <= 16 && EPB == 1;
+}
+
+template <class P, int NQ, bool CVEL, class Args>
+int launch_small(const Args &a, hipStream_t s) {
+  using C = Seq<P, NQ>;
+  static_assert(C::LDS_BYTES_ONCE <= 64 * 1024, "no attribute to set");
+  hipLaunchKernelGGL((stage_small<P, NQ, CVEL>), dim3((unsigned)a.Ne), dim3(C::THREADS),
+                     C::LDS_BYTES_ONCE, s, a.q, a.q0, a.u, a.v, a.w, a.out, a.nbr, a.vmapP, a.D, a.ell,
+                     a.geo, a.geoid, a.order, a.Ne, a.ca, a.cb, a.dt, a.mode, a.axis_aligned,
+                     a.dt_geo, a.reverse, a.zperiod);
+  DGK_HIP(hipGetLastError());
+  return DGK_OK;
+}
+
 template <class P, int NQ, int EPB, bool SEQ, class Args>
 int launch_shape(const Args &a, hipStream_t s) {
   constexpr bool AXR = ax_runtime<P, NQ, EPB, SEQ>();
   // constant velocity: batched and served boxes, whose faces are axis-aligned
-  if (a.cvel && a.axis_aligned && !a.vmapP)
+  const bool cvel = a.cvel && a.axis_aligned && !a.vmapP;
+  if constexpr (has_small<P, NQ, EPB>())
+    if (a.Ne <= (cvel ? 2 * kCus : kCus))
+      return cvel ? launch_small<P, NQ, true>(a, s) : launch_small<P, NQ, false>(a, s);
+  if (cvel)
     return launch_form<P, NQ, EPB, SEQ, !AXR, Args, true>(a, s);
   if constexpr (!AXR)
     if (a.axis_aligned) return launch_form<P, NQ, EPB, SEQ, true>(a, s);

@@ -166,7 +166,9 @@ def kernel_name(evaltype, p: int, cand: int, axis_aligned: bool = True,
     (batches of constant-velocity instances, served requests); the last
     template argument marks a workgroup of several elements reading one
     geometry record for the whole launch (single meshes and served requests,
-    not batches, whose instances have records of their own)."""
+    not batches, whose instances have records of their own).  Mixed launches of
+    at most 256 elements (512 with a constant velocity) at p = 13..15 run
+    stage_small whatever the candidate of one element."""
     if isinstance(evaltype, str):
         evaltype = evaltype_id(evaltype)
     nq = p + 1
