@@ -7,7 +7,10 @@ from seed 2, dt from CFL 0.1.  A "step" is one SSP-RK3 time step of the whole
 mesh (3 fused stage kernels).  Inputs are resident in HBM before the timed
 region.  Metric: DOF-updates/s = Ne*Np*K / t for K timed steps.
 
-The JSON line also carries
+The printed line holds the figures below without the long lists (the per-order
+rows as one time per order and form, no per-request and per-shape lists), so that
+it stays under MAX_LINE bytes; --detail FILE writes the whole record there.  It
+carries
   roofline      the FP64 stage kernel: algorithmic HBM bytes per launch
                 (64/3 B per DOF, the wind being constant; 136/3 B with
                 DGK_CVEL=0) over its average launch time, from HIP events
@@ -53,6 +56,7 @@ HBM_PEAK_GBS = 8000.0
 CONSTANT_WIND = os.environ.get("DGK_CVEL", "1")[:1] != "0"
 BYTES_PER_DOF_UPDATE = ({"HIP": 64.0, "HIP_MP": 64.0} if CONSTANT_WIND
                         else {"HIP": 136.0, "HIP_MP": 100.0})
+MAX_LINE = 6000
 METRIC = "DOF-updates/s plain FP64 vs batched mixed-prec; p50/p99 solve latency"
 
 
@@ -75,6 +79,8 @@ def parse():
                     help="arrival rate of the serving stream, requests/s")
     ap.add_argument("--serve-burst", type=int, default=60,
                     help="requests submitted at once to measure serving capacity (0: skip)")
+    ap.add_argument("--detail", type=Path, default=None, metavar="FILE",
+                    help="also write the whole record, with every list, to FILE")
     ap.add_argument("--per-order-only", type=int, default=0, metavar="P",
                     help="only run --steps steps of the per-order workload at order P "
                          "(periodic box of about 1.7e7 DOF, default tile shape, --form) "
@@ -446,10 +452,11 @@ def c3_leg(dgk, inputs):
             s.synchronize()
             t1 = time.perf_counter()
             fields[form] = s.get_field(dgk.FIELD_Q)
+            tile = s.tile()
         out[form] = {"DOF-updates/s": dof * wl.nstep / (t1 - t0),
                      "ms_per_step": 1e3 * (t1 - t0) / wl.nstep,
-                     "elements_per_workgroup": dgk.tile_shapes(form, wl.p)[dgk.tile_selected(form, wl.p)],
-                     "tile_candidate": dgk.tile_selected(form, wl.p)}
+                     "elements_per_workgroup": dgk.tile_shapes(form, wl.p)[tile],
+                     "tile_candidate": tile}
     ref, mp = fields["HIP"], fields["HIP_MP"]
     out["mp_rel_l2_vs_fp64"] = float(np.linalg.norm(mp - ref) / np.linalg.norm(ref))
     out["mp_max_rel_vs_fp64"] = float(np.abs(mp - ref).max() / np.abs(ref).max())
@@ -499,14 +506,59 @@ def cpu_baseline(wl, steps):
             "cores": oracle.num_threads(), "kind": "port", "sample": sample, "runs": runs}
 
 
+def rounded(x, digits=6):
+    """x with every float to `digits` significant digits."""
+    if isinstance(x, float):
+        return float(f"{x:.{digits}g}")
+    if isinstance(x, dict):
+        return {k: rounded(v, digits) for k, v in x.items()}
+    if isinstance(x, list):
+        return [rounded(v, digits) for v in x]
+    return x
+
+
+def short_line(full):
+    """The printed line: the record with its lists and notes left out or folded.
+    The top-level numbers are those of the record, unrounded."""
+    line = dict(full)
+    roof = dict(full["roofline"])
+    for key in ("timing", "autotune_us_per_launch"):
+        roof.pop(key, None)
+    line["roofline"] = rounded(roof)
+    if full.get("cpu_baseline"):
+        line["cpu_baseline"] = rounded({k: v for k, v in full["cpu_baseline"].items()
+                                        if k not in ("runs", "port_same_inputs", "one_core")})
+    extra = {k: v for k, v in full["extra"].items() if k != "device_timers"}
+    if "batched_ensemble" in extra:
+        be = extra["batched_ensemble"]
+        extra["batched_ensemble"] = {
+            **{k: be[k] for k in ("instances", "nstep", "speedup_batched_mp_vs_plain_fp64_p7")},
+            **{k: v["DOF-updates/s"] for k, v in be.items()
+               if isinstance(v, dict) and "DOF-updates/s" in v},
+            "max_rel_l2_mp_vs_fp64": be["per_instance_mp_vs_fp64"]["max_rel_l2"]}
+    if "per_order" in extra:
+        extra["per_order_us_per_launch"] = {
+            form: {str(r["p"]): round(r["avg_launch_us"], 1) for r in extra["per_order"]
+                   if r["form"] == form} for form in ("HIP", "HIP_MP")}
+        del extra["per_order"]
+    if "serving" in extra:
+        sv = extra["serving"]
+        extra["serving"] = {
+            **{k: sv[k] for k in ("requests", "rate_per_s", "DOF-updates/s", "makespan_s")},
+            "capacity_burst": sv.get("capacity_burst"),
+            "sample_vs_alone": {k: v for k, v in (sv.get("sample_vs_alone") or {}).items()
+                                if k != "requests"}}
+    line["extra"] = rounded(extra)
+    return line
+
+
 def main():
     args = parse()
     if args.copy_calibration:
         copy_calibration(args.copy_calibration)
         return
     if args.gpus != 1:
-        print(json.dumps({"error": "this build runs on one GPU only; a multi-GPU layout is "
-                                   "described in DESIGN.md, not provided as a run mode"}))
+        print(json.dumps({"error": "one GPU only: a multi-GPU run mode is not provided"}))
         sys.exit(2)
     import dgk
     if args.stream_calibration:
@@ -598,8 +650,10 @@ def main():
         try:
             line["cpu_baseline"] = cpu_baseline(wl, args.cpu_steps)
         except Exception as exc:  # reported, never silently replaced
-            line["cpu_baseline"] = {"error": str(exc)}
-    print(json.dumps(line), flush=True)
+            line["cpu_baseline"] = {"error": str(exc)[:500]}
+    if args.detail:
+        args.detail.write_text(json.dumps(line) + "\n")
+    print(json.dumps(short_line(line)), flush=True)
 
 
 if __name__ == "__main__":
