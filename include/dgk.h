@@ -117,9 +117,9 @@ int dgk_mesh_build(int NeX, int NeY, int NeZ, int p, const double *x1D,
  * Processing order (never the arithmetic, so never the results): a mesh
  * numbered plane by plane along z with periodic +z neighbours and planes of
  * at least 8 elements is dealt to the GPU's 8 XCDs in eighths of every
- * plane (XCD x walks the eighth x of every plane in turn; the FP64 VALU
- * kernels keep the element numbering where an eighth holds fewer than 96
- * elements), and consecutive stage launches walk the elements in opposite
+ * plane (XCD x walks the eighth x of every plane in turn; the staged and
+ * general-normal FP64 VALU kernels keep the element numbering where an eighth
+ * holds fewer than 96 elements), and consecutive stage launches walk the elements in opposite
  * directions (each XCD its own elements, in that order).  Environment:
  * DGK_ORDER=identity keeps the element numbering, DGK_ALT=0 keeps one
  * direction, DGK_ALT=global reverses the whole order instead
@@ -207,7 +207,7 @@ int dgk_minmax_noalloc(const double *q, int64_t n, double *result, void *stream)
 
 /* ---- timers (mod_common.f90:33-71, names of main.f90:175-177 and
  * mod_advect3d_eq.f90:34-35) ---------------------------------------------
- * seconds[0] Main (host wall time inside dgk_step),
+ * seconds[0] Main (device time of dgk_step, from HIP events around its launches),
  * seconds[1] Cal_tend (device time of tendency kernels),
  * seconds[2] Element boundary flux (device, dgk_cal_elembnd_flux),
  * seconds[3] Volume derivate + surface lift (device, dgk_cal_dqdt),
@@ -295,7 +295,7 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * itself runs direction-by-direction launches of the mixed form at p = 16, 17,
  * constant-velocity ones of the mixed form at p >= 16 and of FP64 at p = 16, and
  * the mixed form's launches of at most 256 elements (512 with a constant
- * velocity) at p = 13..15, all at once, whatever the candidate.
+ * velocity) at p = 13..15, all at once, for either candidate of one element.
  * dgk_tile_select sets the process-wide choice for that form and order, for
  * both kinds of launch (-1 restores the defaults); it holds for every solver
  * that has not been autotuned; dgk_tile_selected reports the choice for
@@ -303,10 +303,10 @@ int dgk_batch_timer(dgk_batch *b, double *seconds, int64_t *calls);
  * or a stored, non-separable Lift always use the VALU kernels.  dgk_autotune
  * times each candidate with HIP events over the stage launches of whole steps,
  * at least reps of them, on the solver's own mesh (writing only its scratch
- * rotation buffers) and
- * keeps the fastest for that solver alone, since the best shape depends on
- * the mesh (the solver's default stays unless another shape is at least 2%
- * faster);
+ * rotation buffers) and keeps the fastest for that solver alone, since the best
+ * shape depends on the mesh (the solver's default stays unless another shape is
+ * at least 2% faster), and for the kind of launch that the solver has then (with
+ * velocity fields or a constant velocity);
  * us_per_launch[c] receives candidate c's time (0 for a candidate that would
  * launch another shape on this solver: the kernel over runs of elements, on
  * launches it cannot take -- batches' constant velocities, a resolved face-node
@@ -352,7 +352,7 @@ enum { DGK_TOL_FP64 = 0, /* plain FP64 path (HIP)                         */
 
 typedef struct dgk_request {
   int32_t ne[3];     /* elements per axis (>= 1)                           */
-  int32_t p;         /* polynomial order 1..15                             */
+  int32_t p;         /* polynomial order 1..19                             */
   int32_t nstep;     /* SSP-RK3 steps (>= 0)                               */
   int32_t tol_class; /* DGK_TOL_FP64 or DGK_TOL_1E5                        */
   double dom[3];     /* box size per axis (> 0)                            */

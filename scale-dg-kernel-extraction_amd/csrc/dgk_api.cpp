@@ -36,7 +36,9 @@ hipEvent_t take_event(dgk_solver *s) {
     return e;
   }
   hipEvent_t e = nullptr;
-  // timing only: without the fence to system scope that a default event brings
+  // Timing only: without the fence to system scope that a default event brings.
+  // What is read is the event's own time stamps, here by a query or after a wait for
+  // the stream; no caller takes an event for the memory written before it.
   if (hipEventCreateWithFlags(&e, hipEventDisableSystemFence) != hipSuccess) return nullptr;
   return e;
 }
@@ -157,8 +159,8 @@ static int geo_velocity_from_field(dgk_solver *s, int d) {
 // The kind of the solver's stage launches after a change of its velocity
 // fields: constant components on axis-aligned faces are read from the
 // geometry records, 64 bytes per DOF-update instead of 136 (FP64) or 100
-// (mixed), with the same bits (at 32^3, p = 7: 139 -> 101 us per launch FP64,
-// 102 -> 94 us mixed).  Node connectivity has no such form.  DGK_CVEL=0 keeps
+// (mixed), with the same bits (at 32^3, p = 7: 128 -> 67 us per launch FP64,
+// 94 -> 64 us mixed).  Node connectivity has no such form.  DGK_CVEL=0 keeps
 // the per-node reads (for A/B timings).  A tile shape autotuned for one kind
 // is kept for it.
 static void choose_velocity_form(dgk_solver *s) {

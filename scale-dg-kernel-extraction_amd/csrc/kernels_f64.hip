@@ -19,9 +19,9 @@
 //   2. upwind flux of face node (i,j) of every face from the LDS copy;
 //   3. F = q*(u,v,w) in place in LDS;
 //   With VREG only q and u are staged: the lane loads its v and w columns
-//   (and the v traces of its y faces) into registers, and Fy takes the place
-//   of q.  That halves the LDS per element (more workgroups per CU) for a
-//   few more registers; the arithmetic is the same.
+//   into registers, and Fy takes the place of q.  That halves the LDS per
+//   element (more workgroups per CU) for a few more registers; the arithmetic
+//   is the same.
 //   4. per node: the three sum-factorised contractions from LDS (D rows in
 //      registers), the Lift in tensor-product form -- face f contributes
 //      l-/+(x_n) * flux_f(tangential node) along its normal n, with l-/+ taken
@@ -29,7 +29,8 @@
 //      dqdt = -(((Ex Dx + Ey Dy) + Ez Dz) + Lift), stored or RK-combined.
 //
 // With axis-aligned faces and no given flux the register form (VREG) runs
-// stage_pencil instead: the same arithmetic, a pencil per lane and direction.
+// stage_pencil instead: the same arithmetic, a pencil per lane and direction.  A
+// given flux runs it as stage_f64_flux, other normals as stage_f64.
 //
 // stage_f64_lift<NQ> (stored Lift): the same arithmetic with Lift_mat read as
 // stored; used when Lift_mat is not of tensor-product form.
@@ -91,12 +92,9 @@ struct Staged {
   // (lane (i,j) writes where lane (j,i) read in the same instruction slot);
   // the x-contraction then reads consecutive addresses.
   static constexpr bool FX_T = WAVES == 1;
-  // Waves per SIMD the register allocation must leave room for: 3 for the
-  // register form at p = 11, which otherwise lands one VGPR above the
-  // 168 that 3 waves allow (and drops to 2).
-  static constexpr int MIN_WAVES_EU = (VREG && NQ == 12) ? 3 : 1;
-  // The given-flux kernel: 5 waves at p = 4 (108 VGPRs -> 96 or fewer; 153 ->
-  // 147 us per launch) and 3 at p = 13 (186 -> 168 with 6 spilled; 196 -> 172).
+  // Waves per SIMD that the given-flux kernel's register allocation must leave room
+  // for: 5 at p = 4 (108 VGPRs -> 96 with 6 spilled; 153 -> 147 us per launch) and 3
+  // at p = 13 (186 -> 168 with 6 spilled; 196 -> 172).
   static constexpr int MIN_WAVES_EU_FLUX = NQ == 14 ? 3 : NQ == 5 ? 5 : 1;
 };
 
@@ -105,7 +103,7 @@ struct Staged {
 // other components enter the normal velocity as exact zeros).  The general
 // form holds three more traces per face in registers; a compile-time choice
 // lets the axis-aligned kernel drop them (p = 1: 85 -> 62 VGPRs, 5 -> 8 waves
-// per SIMD).  The axis-aligned register forms run stage_pencil instead.
+// per SIMD).  The axis-aligned register form is stage_pencil.
 // CVEL: every element's velocity is constant, (u, v, w) = words kGeoVel..+2
 // of its geometry record (batched and served boxes); no velocity field is
 // read.  The constants enter the same expressions as the per-node values
@@ -132,6 +130,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
   // Read-only operands are __restrict__ kernel parameters, so wave-uniform
   // reads of them (operators, geometry, neighbour table) are scalar loads.
   static_assert(!CVEL || AXAL, "constant velocity on axis-aligned faces");
+  static_assert(!VREG || !AXAL, "stage_pencil is the axis-aligned register form");
   constexpr bool F64_VEL = std::is_same<VT, double>::value;
   static_assert(F64_VEL || VREG, "FP32 velocities: the register form only");
   using C = Staged<NQ, VREG>;
@@ -204,7 +203,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
         src[2] = v_;
         src[3] = w_;
       }
-      constexpr int NASYNC = (CVEL || !F64_VEL) ? 1 : C::NSTAGED;
+      constexpr int NASYNC = CVEL || !F64_VEL ? 1 : C::NSTAGED;
 #pragma unroll
       for (int c0 = 0; c0 < C::NCHUNK; c0 += C::WAVES) {
         const int c = c0 + wave;
@@ -235,7 +234,7 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
 
     // FP32 velocities: this lane's u column, as doubles, into the staged u
     // field at the slots the async copy would fill
-    if constexpr (!F64_VEL && !CVEL) {
+    if constexpr (!F64_VEL) {
       if (active) {
 #pragma unroll
         for (int k = 0; k < NQ; ++k) su[lb + ij + k * NQ2] = (double)u_[base + (int64_t)k * NQ2];
@@ -274,16 +273,16 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
         }
       }
     }
-    // VREG: the v and w columns and the v traces of the y faces
-    double vc[VREG ? NQ : 1], wc[VREG ? NQ : 1], vM[2];
-    if (VREG && active) {
+    // VREG: the v and w columns
+    double vc[VREG ? NQ : 1], wc[VREG ? NQ : 1];
+    if constexpr (VREG) {
+      if (active) {
 #pragma unroll
-      for (int k = 0; k < NQ; ++k) {
-        vc[k] = CVEL ? cvel[1] : v_[base + (int64_t)k * NQ2];
-        wc[k] = CVEL ? cvel[2] : w_[base + (int64_t)k * NQ2];
+        for (int k = 0; k < NQ; ++k) {
+          vc[k] = v_[base + (int64_t)k * NQ2];
+          wc[k] = w_[base + (int64_t)k * NQ2];
+        }
       }
-      vM[0] = CVEL ? cvel[1] : v_[e * NP + own_face_node(0, i, j, NQ)];
-      vM[1] = CVEL ? cvel[1] : v_[e * NP + own_face_node(2, i, j, NQ)];
     }
     // the RK base and the output are touched once per launch: non-temporal,
     // so L2 keeps the neighbour traces -- where a k-slab of an element is a
@@ -323,9 +322,6 @@ stage_valu(const double *__restrict__ q_, const double *q0_, const VT *__restric
             double vm;
             if constexpr (CVEL)
               vm = cvel[kFaceAxis[f]];
-            else if constexpr (VREG)
-              vm = kFaceAxis[f] == 0 ? su[m] : f == 0 ? vM[0] : f == 2 ? vM[1]
-                   : f == 4 ? wc[0] : wc[NQ - 1];
             else
               vm = (kFaceAxis[f] == 0 ? su : kFaceAxis[f] == 1 ? sv : sw)[m];
             const double na = g[kGeoNormal + 3 * f + kFaceAxis[f]];
@@ -678,7 +674,7 @@ stage_pencil(const double *__restrict__ q_, const double *q0_, const VT *__restr
 template <int NQ, bool VREG, bool AXAL, bool CVEL, bool GU>
 __global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, VREG>::THREADS),
                                amdgpu_waves_per_eu(VREG && AXAL ? Pencil<NQ, CVEL>::MIN_WAVES_EU
-                                                                : Staged<NQ, VREG>::MIN_WAVES_EU)))
+                                                                : 1)))
 stage_f64(const double *__restrict__ q_, const double *q0_, const double *__restrict__ u_,
           const double *__restrict__ v_, const double *__restrict__ w_, double *out_,
           const double *__restrict__ flux_in_, const int32_t *__restrict__ nbr_,
@@ -722,8 +718,7 @@ stage_f64_flux(const double *__restrict__ q_, const double *q0_, const double *_
 // The mixed form's VALU kernel (register form, FP32 velocity fields).
 template <int NQ, bool AXAL, bool CVEL, bool GU>
 __global__ void __attribute__((amdgpu_flat_work_group_size(1, Staged<NQ, true>::THREADS),
-                               amdgpu_waves_per_eu(AXAL ? Pencil<NQ, CVEL>::MIN_WAVES_EU
-                                                        : Staged<NQ, true>::MIN_WAVES_EU)))
+                               amdgpu_waves_per_eu(AXAL ? Pencil<NQ, CVEL>::MIN_WAVES_EU : 1)))
 stage_f64_mp(const double *__restrict__ q_, const double *q0_, const float *__restrict__ u_,
              const float *__restrict__ v_, const float *__restrict__ w_, double *out_,
              const int32_t *__restrict__ nbr_, const int32_t *__restrict__ vmapP_,
@@ -1260,32 +1255,35 @@ unsigned grid1d(int64_t n, int threads) {
 }  // namespace
 
 // FP64 tile shapes: candidate 0 is the VALU kernel with q, u, v, w staged in
-// LDS, 1 the VALU kernel with v, w in registers (VREG), 2.. the FP64 MFMA
-// kernel's shapes (kernels_mfma.hip); above p = 15 only the MFMA shapes.  The
-// MFMA kernel computes the flux itself and applies the separable Lift, so
+// LDS, 1 the VALU kernel with v, w in registers (VREG; stage_pencil on
+// axis-aligned faces), 2.. the shapes over augmented pencils (stage_aug.hpp),
+// named after the MFMA; above p = 15 only those.  They compute the flux
+// themselves and apply the separable Lift, so
 // launches that pass a flux (cal_dqdt) or need the stored Lift take the VALU
 // kernels (stage_f64 / stage_f64_lift).
 constexpr int kValuShapes = 2;
-// Default per Nq, from whole-step timings of every candidate on MI355X at
-// about 1.7e7 DOF: the register VALU kernel at p = 4 and 6..13, the
-// direction-by-direction MFMA kernel (the last candidate) at p = 14..19, the
-// staged VALU kernel else (p = 3: 158 -> 153 us per launch once both read a
-// launch-wide geometry record through the scalar cache).  At p = 16, 17 the
-// one-element all-at-once MFMA kernel is candidate 0 (313 and 260 us per
-// launch against 276 and 249 direction by direction: at Nq = 17 its GEMMs
-// take two 16-wide column tiles).
+// Default per Nq: the register (pencil) kernel at p = 4 and 6..13, the
+// direction-by-direction shape (the last candidate) at p = 14..19, the staged
+// kernel else.  us per launch at about 1.7e7 DOF with velocity fields, staged
+// against register form: p = 3 150/146, p = 5 168/165 (level: the default stays),
+// p = 4 164/158, p = 7 166/128, p = 12 234/151; register form against the last
+// candidate: p = 13 152.8/152.0, p = 14 155/150, p = 15 145/141.  The shapes over
+// augmented pencils add in another order, so they are no default below p = 14 (p = 5
+// 153 against 168, elsewhere within 3%).  Above p = 15 all at once and direction by
+// direction are one kernel with fields.
 constexpr int kF64Default[kMaxNq + 1] = {0, 0, 0, 0, 0, 1, 0, 1, 1, 1, 1, 1, 1, 1, 1, 3, 3,
                                          1, 1, 0, 0};
 // Selected FP64 tile shape per Nq (see stage_f64_shapes); atomic because a
 // serving worker may launch while another thread selects.
 std::atomic<int> g_f64_shape[kMaxNq + 1] = {0, 0, 0, 0, 0, 1, 0, 1, 1, 1, 1, 1, 1, 1, 1,
                                             3, 3, 1, 1, 0, 0};
-// Defaults of constant-velocity launches (batches, served requests), from the
-// same timings with the velocity read from the geometry record: the register
-// VALU (pencil) kernel at every p <= 13 (one batched box against the staged
-// kernel: p = 1 183 -> 161, p = 3 158 -> 128, p = 5 142 -> 99 us per launch).
-// Only shapes that give the bits of the default above are taken, so a served
-// request equals its solve on a plain solver.
+// Defaults of constant-velocity launches (batches, served requests, solvers with
+// constant fields): the register (pencil) kernel at every p <= 13 (staged against
+// pencil, a solver: p = 1 108/92, p = 3 107/71, p = 5 131/83, p = 7 131/67 us per
+// launch).  Only shapes that give the bits of the default above are taken, so a
+// served request equals its solve on a plain solver.  At p = 16 the last
+// candidate's product is on the MFMA (146 -> 123), at p = 17..19 it is the other
+// candidate's kernel.
 constexpr int kF64DefaultCvel[kMaxNq + 1] = {0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 3, 3,
                                              1, 1, 0, 0};
 std::atomic<int> g_f64_shape_cvel[kMaxNq + 1] = {0, 0, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1, 1,

@@ -335,17 +335,14 @@ int launch_run_mp(int Nq, const StageArgsMP &a, hipStream_t s) {
   }
 }
 
-// Tile-shape candidate selected per Nq for the mixed form.  Defaults from
-// per-order timings on MI355X at about 1.7e7 DOF (whole-step runs, every
-// candidate, with a launch-wide geometry record read through the scalar
-// cache): the VALU kernel at p = 1 (154 -> 149 us per launch against one
-// wavefront of MFMA tiles; level at p = 2, slower above), the two-wavefront
-// shape at p = 4, the four-wavefront shape at
-// p = 5 (136 -> 126 us per launch), the direction-by-direction shape at
-// p = 14, 16, 17 (p = 16: 203 -> 157 us, p = 17: 163 -> 138 us against one
-// element all at once), the one-wavefront shape else (p = 2: 178 -> 174 us,
-// p = 3: 133 -> 121 us against two wavefronts; p = 18: 165 -> 160 us,
-// p = 19: 193 -> 177 us against direction by direction).
+// Tile-shape candidate selected per Nq for the mixed form: the VALU kernel (FP64
+// arithmetic) at p = 1, two wavefronts at p = 4, four at p = 5, direction by
+// direction at p = 14, 16, 17, one wavefront or element else.  us per launch at about
+// 1.7e7 DOF with velocity fields: p = 1 130 (130 for the others), p = 4 115 for
+// every shape, p = 5 one, two, four wavefronts 115.6/114.0/113.5.  Direction by
+// direction is the same kernel but for its test of the face normals, which is made
+// at run time (p = 11 95.3/100.8, p = 14 106.3/106.8, p = 19 159/164), and the MFMA at
+// p = 16, 17 (172 -> 141, 156 -> 135).
 constexpr int kMpDefault[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
                                         0, 0, 0, 0, 2, 0, 1, 1, 0, 0};
 std::atomic<int> g_mp_shape[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
@@ -353,11 +350,11 @@ std::atomic<int> g_mp_shape[kMaxNq + 1] = {0, 0, 5, 0, 0, 1, 2, 0, 0, 0, 0,
 // Defaults of constant-velocity launches (batches, served requests, solvers with
 // constant fields), from the same timings with the velocity read from the
 // geometry record, among the shapes that give the bits of the default above
-// (all but the VALU kernel), so a served request equals its solve on a plain
-// solver: two wavefronts at p = 4 (59 against 64 us per launch with one), four
-// at p = 5 (75 against 85 on a solver, 84 against 89 on a batched box), one
-// (direction by direction: the same kernel) else; above p = 15 direction by
-// direction, on the MFMA.
+// (all but the VALU kernel, which is the default of both kinds at p = 1), so a
+// served request equals its solve on a plain solver: two wavefronts at p = 4 (71.9
+// against 74.2 us per launch with one), four at p = 5 (71.3 against 77.9), one
+// (direction by direction: the same machine code) else; above p = 15 direction by
+// direction, on the MFMA (p = 16 135 -> 100, p = 19 126 -> 109).
 constexpr int kMpDefaultCvel[kMaxNq + 1] = {0, 0, 5, 3, 3, 1, 2, 3, 3, 2, 2,
                                             2, 2, 2, 2, 2, 2, 1, 1, 1, 1};
 std::atomic<int> g_mp_shape_cvel[kMaxNq + 1] = {0, 0, 5, 3, 3, 1, 2, 3, 3, 2, 2,

@@ -38,7 +38,7 @@
 //  * the MFMA one, direction by direction through one LDS area, where it is
 //    faster (by_mfma): mixed p = 16, 17 (fields 140 against 177 and 137 against
 //    158) and constant-velocity launches of the mixed form at p >= 16 (101
-//    against 139, 104/127, 100/113, 110/130) and of FP64 at p = 16 (133/150).
+//    against 139, 104/127, 100/113, 110/130) and of FP64 at p = 16 (123/146),
 //    and launches of few elements of the mixed form at p = 13..15 (stage_small).
 //    Above p = 15 an element is five to seven wavefronts, and on four SIMDs the VALU
 //    form's phases take as long as two of them, while the MFMA form's eight
@@ -152,7 +152,10 @@ struct Shape {
   static constexpr int THREADS = MFMA ? Seq<P, NQ>::THREADS : Aug<P, NQ, EPB, CVEL>::THREADS;
   static constexpr size_t LDS_BYTES =
       MFMA ? Seq<P, NQ>::LDS_BYTES : Aug<P, NQ, EPB, CVEL>::LDS_BYTES;
-  static constexpr int MIN_WAVES_EU = MFMA ? 4 : 1;
+  // 4 waves per SIMD also for the mixed constant-velocity form at p = 15, which
+  // lands at 131 VGPRs otherwise (73.2 -> 71.7 us per launch)
+  static constexpr int MIN_WAVES_EU =
+      MFMA || (CVEL && NQ == 16 && EPB == 1 && sizeof(typename P::op_t) == 4) ? 4 : 1;
 };
 
 // Shapes whose face normals are tested at run time, in one instantiation for
@@ -166,12 +169,12 @@ constexpr bool ax_runtime() {
 // Candidate kinds per order: for Nq^2 <= 64 one, two or four wavefronts of
 // whole elements, then one wavefront direction by direction; above, one
 // element, two elements, and one element direction by direction; above
-// p = 15 one element, all at once or direction by direction.  Kinds whose A
-// (three areas all at once, one direction by direction) would exceed a CU's
-// 160 KiB of LDS are dropped (all at once above p = 15: FP64 up to p = 17,
-// mixed up to p = 19); the remaining ones are the candidates 0, 1, ...
-// (per-order defaults in kMpDefault below).  In the VALU form all at once and
-// direction by direction are the same kernel.
+// p = 15 one element, all at once or direction by direction.  The candidates
+// 0, 1, ... are the kinds of an order that kind_ok keeps (per-order defaults in
+// kMpDefault and kF64Default).  In the VALU form all at once and direction by
+// direction are one algorithm; the second tests the face normals at run time where
+// velocity fields are read (with a constant velocity they are the same machine code).
+// Both stay: candidates are numbered and selected by callers.
 constexpr int kKinds = 4;
 template <int NQ>
 constexpr int kind_epb(int k) {
@@ -187,6 +190,10 @@ template <int NQ>
 constexpr bool kind_seq(int k) {
   return NQ * NQ > 64 ? k == 2 : k == 3;
 }
+// The kinds an order has.  The last line is the LDS that three areas of A all at once
+// (one direction by direction) take on the MFMA, which the VALU form does not
+// allocate: it keeps the candidates' numbers what they have been (all at once above
+// p = 15: FP64 up to p = 17, mixed up to p = 19).
 template <class P, int NQ>
 constexpr bool kind_ok(int k) {
   if (NQ * NQ > 64 && k == 3) return false;
@@ -296,7 +303,7 @@ stage_aug(const double *__restrict__ q_, const double *q0_,
   const int64_t ebase = e * NP, base = ebase + ij;
   const bool rk = mode_ == 1;
   const bool use_q0 = rk && ca_ != 0.0;
-  const bool axal = AXR ? axis_aligned_ != 0 : AXAL;
+  const bool axal = CVEL || (AXR ? axis_aligned_ != 0 : AXAL);  // launch_shape
 
   double qc[NQ], qP[6], q0v[NQ];
   vel_t vP[6], uc[NQ], vc[NQ], wc[NQ];
@@ -377,15 +384,8 @@ stage_aug(const double *__restrict__ q_, const double *q0_,
                                     : (int64_t)nbr_[e * 6 + f] * NP + nbr_face_node(f, i, j, NQ);
         const double n1 = g[kGeoNormal + 3 * f], n2 = g[kGeoNormal + 3 * f + 1],
                      n3 = g[kGeoNormal + 3 * f + 2];
-        if constexpr (CVEL) {
-          VelM = (double)cv[0] * n1 + (double)cv[1] * n2 + (double)cv[2] * n3;
-          VelP = VelM;
-          (void)m;
-          (void)pidx;
-        } else {
-          VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
-          VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
-        }
+        VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
+        VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
       }
       const double alpha = 0.5 * fabs(VelP + VelM);
       return (op_t)(0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qm * VelM - alpha * (qP[f] - qm)));
@@ -546,7 +546,7 @@ stage_seq(const double *q_, const double *q0_,
   const int64_t base = ebase + ij;
   const bool rk = mode_ == 1;
   const bool use_q0 = rk && ca_ != 0.0;
-  const bool axal = axis_aligned_ != 0;
+  const bool axal = CVEL || axis_aligned_ != 0;  // launch_shape
   const vel_t *const velp[3] = {u_, v_, w_};
   vel_t cv[3] = {(vel_t)0, (vel_t)0, (vel_t)0};
   if constexpr (CVEL) {
@@ -608,15 +608,8 @@ stage_seq(const double *q_, const double *q0_,
       const int64_t pidx = nbr_at(f);
       const double n1 = g[kGeoNormal + 3 * f], n2 = g[kGeoNormal + 3 * f + 1],
                    n3 = g[kGeoNormal + 3 * f + 2];
-      if constexpr (CVEL) {
-        VelM = (double)cv[0] * n1 + (double)cv[1] * n2 + (double)cv[2] * n3;
-        VelP = VelM;
-        (void)m;
-        (void)pidx;
-      } else {
-        VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
-        VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
-      }
+      VelM = (double)u_[m] * n1 + (double)v_[m] * n2 + (double)w_[m] * n3;
+      VelP = (double)u_[pidx] * n1 + (double)v_[pidx] * n2 + (double)w_[pidx] * n3;
     }
     const double alpha = 0.5 * fabs(VelP + VelM);
     fl[f] = (op_t)(0.5 * g[kGeoFscale + f] * (qP[f] * VelP - qm * VelM - alpha * (qP[f] - qm)));
@@ -888,7 +881,7 @@ int launch_small(const Args &a, hipStream_t s) {
 template <class P, int NQ, int EPB, bool SEQ, class Args>
 int launch_shape(const Args &a, hipStream_t s) {
   constexpr bool AXR = ax_runtime<P, NQ, EPB, SEQ>();
-  // constant velocity: batched and served boxes, whose faces are axis-aligned
+  // constant velocity: on axis-aligned faces only
   const bool cvel = a.cvel && a.axis_aligned && !a.vmapP;
   if constexpr (has_small<P, NQ, EPB>())
     if (a.Ne <= (cvel ? 2 * kCus : kCus))

@@ -22,8 +22,9 @@ constexpr int64_t kChunk = (int64_t)1 << 20;    // bytes of a pinned chunk
 // Below this a plain copy is as fast as starting the threads (16.8 MB: 1.2 ->
 // 0.8 ms, 134 MB: 12.8 -> 4.2 ms, the caller's pages fresh in both).
 constexpr int64_t kSliced = (int64_t)4 << 20;
-// Making the pool takes 3-4 ms, which plain copies lose against sliced ones
-// over about this many bytes.
+// Making the pool takes 7-8 ms with its streams' first use, of which a first plain
+// copy pays most as well: a first download of 57 MB 16.5 ms sliced, 17.2 plain, of
+// 134 MB 18.9 and 24.8.  Below this many bytes a program is left with plain copies.
 constexpr int64_t kWorthPool = (int64_t)48 << 20;
 
 // The pinned chunks, streams and events of one download at a time, shared by

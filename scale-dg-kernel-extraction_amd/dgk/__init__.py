@@ -168,7 +168,8 @@ def kernel_name(evaltype, p: int, cand: int, axis_aligned: bool = True,
     geometry record for the whole launch (single meshes and served requests,
     not batches, whose instances have records of their own).  Mixed launches of
     at most 256 elements (512 with a constant velocity) at p = 13..15 run
-    stage_small whatever the candidate of one element."""
+    stage_small for either candidate of one element, and launches from a given
+    flux stage_f64_flux where candidate 1 is selected."""
     if isinstance(evaltype, str):
         evaltype = evaltype_id(evaltype)
     nq = p + 1
