@@ -10,8 +10,20 @@ pytestmark = pytest.mark.gpu
 
 VEL = (0.3, -0.7, 0.5)
 # timings of one kernel differ by 3%, the faults below by 20% and more; each
-# figure is the least of three, an interrupted sequence takes longer
+# figure is the least of three and a pair that disagrees is measured again, since
+# something else may have held the device meanwhile
 WITHIN = 0.10
+ATTEMPTS = 3
+
+
+def agree(pair):
+    seen = []
+    for _ in range(ATTEMPTS):
+        tuned, step = pair()
+        seen.append((tuned, step))
+        if abs(tuned - step) < WITHIN * step:
+            return
+    raise AssertionError(seen)
 
 
 @pytest.mark.parametrize("form,p,ne", [("HIP", 7, 32), ("HIP", 3, 64), ("HIP_MP", 7, 32)])
@@ -20,19 +32,24 @@ def test_solver_times_are_the_steps(form, p, ne):
         s.init_gaussian((0.3, 0.4, 0.5), 0.1, VEL)
         s.step(1e-5, 30)
         before = s.get_field(dgk.FIELD_Q)
-        runs = [s.autotune(60) for _ in range(3)]
-        assert (s.get_field(dgk.FIELD_Q) == before).all()
-        best = runs[-1]["best"]
-        tuned = min(r["us_per_launch"][best] for r in runs)
-        steps = []
-        for _ in range(3):
+
+        def tuned():
+            runs = [s.autotune(60) for _ in range(3)]
+            best = runs[-1]["best"]
+            return min(r["us_per_launch"][best] for r in runs)
+
+        def step():
             s.timer_reset()
             s.set_kernel_timing(True)
             s.step(1e-5, 40)
             s.synchronize()
+            s.set_kernel_timing(False)
             seconds, n = s.timers()["Stage (fused)"]
-            steps.append(1e6 * seconds / n)
-    assert abs(tuned - min(steps)) < WITHIN * min(steps), (steps, runs)
+            return 1e6 * seconds / n
+
+        tuned()
+        assert (s.get_field(dgk.FIELD_Q) == before).all()
+        agree(lambda: (tuned(), min(step() for _ in range(3))))
 
 
 @pytest.mark.parametrize("form,p,ne", [("HIP_MP", 2, 85), ("HIP", 3, 64), ("HIP", 7, 32)])
@@ -45,15 +62,24 @@ def test_batch_times_are_the_steps(form, p, ne):
         b.step(20)
         b.synchronize()
         before = b.get_field(0)
-        runs = [b.autotune(reps=60) for _ in range(3)]
-        assert (b.get_field(0) == before).all()
-        tuned = min(r[0]["us_per_launch"] for r in runs if r[0]["candidate"] == runs[-1][0]["candidate"])
-        b.step(20)
-        steps = []
-        for _ in range(3):
+
+        def tuned():
+            runs = [b.autotune(reps=60)[0] for _ in range(3)]
+            return min(r["us_per_launch"] for r in runs if r["candidate"] == runs[-1]["candidate"])
+
+        def step():
             b.synchronize()
             b.timer()
             b.step(40)
             seconds, _ = b.timer()
-            steps.append(1e6 * seconds / 120)
-    assert abs(tuned - min(steps)) < WITHIN * min(steps), (steps, runs)
+            return 1e6 * seconds / 120
+
+        tuned()
+        assert (b.get_field(0) == before).all()
+
+        def pair():
+            t = tuned()
+            b.step(20)
+            return t, min(step() for _ in range(3))
+
+        agree(pair)

@@ -62,10 +62,10 @@ def test_default_is_the_register_form(p, ne):
     with dgk.Solver.structured("HIP", ne, ne, ne, p) as s:
         s.init_gaussian((0.3, 0.4, 0.5), 0.1, (0.3, -0.7, 0.5))
         s.cal_elembnd_flux(download=False)
-        default = per_launch(s)
+        default = min(per_launch(s) for _ in range(3))
         try:
             dgk.tile_select("HIP", p, 0)
-            staged = per_launch(s)
+            staged = min(per_launch(s) for _ in range(3))
         finally:
             dgk.tile_select("HIP", p, -1)
     assert default < 0.9 * staged, (default, staged)
